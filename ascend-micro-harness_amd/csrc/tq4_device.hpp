@@ -16,8 +16,6 @@ namespace tq4 {
 
 constexpr int kStrip = 16;            // tokens per strip (R)
 constexpr float kMasked = -3.0e38f;   // score of a masked lane, also the neutral m
-constexpr int kPolicyPrefill = 0;     // absmax floored at 1.0
-constexpr int kPolicyExact = 1;       // exact absmax, zero row -> scale 1.0
 
 __device__ __forceinline__ float bf16_to_f32(uint32_t raw16)
 {

@@ -87,59 +87,6 @@ __device__ __forceinline__ void load_signs(const float* pi_signs, const void* ta
     }
 }
 
-// Rotate one row, find its absmax over the 16 lanes of the row, quantise.
-// q receives the INT4 codes, the return value is the stored scale.
-template <int D, int CPL>
-__device__ __forceinline__ float rotate_quantise(float (&v)[CPL], const float (&sign)[CPL],
-                                                 int lane_in_row, float inv_sqrt_len, int policy,
-                                                 int (&q)[CPL])
-{
-    rotate_ingress<D, CPL>(v, sign, lane_in_row);
-    float a = 0.0f;
-#pragma unroll
-    for (int j = 0; j < CPL; ++j) a = fmaxf(a, fabsf(v[j]));
-#pragma unroll
-    for (int m = 1; m < 16; m <<= 1) a = fmaxf(a, xor_lanes(a, m));
-    if (policy == kPolicyPrefill) {
-        a = fmaxf(a, 1.0f);
-    } else if (a == 0.0f) {
-#pragma unroll
-        for (int j = 0; j < CPL; ++j) q[j] = 0;
-        return 1.0f;
-    }
-    const int e = exponent_of(a);
-#pragma unroll
-    for (int j = 0; j < CPL; ++j) {
-        float r = rintf(ldexpf(v[j], 2 - e));
-        r = fminf(r, 7.0f);
-        q[j] = (int)r;
-    }
-    return ldexpf(1.0f, e - 2) * inv_sqrt_len;
-}
-
-// Pack CPL codes (low nibble first) into CPL/2 bytes and store them.
-template <int CPL>
-__device__ __forceinline__ void store_key_codes(int8_t* dst, const int (&q)[CPL])
-{
-    if constexpr (CPL == 16) {
-        uint32_t w[2] = {0u, 0u};
-#pragma unroll
-        for (int j = 0; j < 16; ++j) w[j / 8] |= ((uint32_t)q[j] & 0xfu) << (4 * (j % 8));
-        *(uint2*)dst = make_uint2(w[0], w[1]);
-    } else if constexpr (CPL == 8) {
-        uint32_t w = 0u;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) w |= ((uint32_t)q[j] & 0xfu) << (4 * j);
-        *(uint32_t*)dst = w;
-    } else {
-        static_assert(CPL == 4, "head_size 64, 128 or 256");
-        uint32_t w = 0u;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) w |= ((uint32_t)q[j] & 0xfu) << (4 * j);
-        *(uint16_t*)dst = (uint16_t)w;
-    }
-}
-
 // ------------------------------------------------------------ strip writer
 // The strip writer's row order and arithmetic, tuned for the VALU issue rate
 // (with two waves per SIMD the writer's rotation, quantisation and packing
@@ -269,6 +216,29 @@ __device__ __forceinline__ uint32_t pack4(const uint32_t* t)
     return (__builtin_amdgcn_perm(p23, p01, 0x0C0C0400u) ^ 0x8888u) & 0xffffu;
 }
 
+// Word w (channel w / 2, token half w % 2) of a strip's value words from the
+// transpose buffer: that channel's codes of tokens 8 * half .. + 7, one nibble
+// of each of 8 consecutive buffer words (two 16-byte reads).
+__device__ __forceinline__ uint32_t strip_word(const uint32_t (*lds_t)[20], int w)
+{
+    const int channel = w >> 1, half = w & 1;
+    const uint32_t* src = &lds_t[channel >> 3][8 * half];
+    const uint4 a = *(const uint4*)src;
+    const uint4 b = *(const uint4*)(src + 4);
+    const uint32_t sh = 4u * (uint32_t)(channel & 7);
+    const uint32_t n[8] = {__builtin_amdgcn_ubfe(a.x, sh, 4), __builtin_amdgcn_ubfe(a.y, sh, 4),
+                           __builtin_amdgcn_ubfe(a.z, sh, 4), __builtin_amdgcn_ubfe(a.w, sh, 4),
+                           __builtin_amdgcn_ubfe(b.x, sh, 4), __builtin_amdgcn_ubfe(b.y, sh, 4),
+                           __builtin_amdgcn_ubfe(b.z, sh, 4), __builtin_amdgcn_ubfe(b.w, sh, 4)};
+    const uint32_t p01 = (n[1] << 4) | n[0];
+    const uint32_t p23 = (n[3] << 4) | n[2];
+    const uint32_t p45 = (n[5] << 4) | n[4];
+    const uint32_t p67 = (n[7] << 4) | n[6];
+    const uint32_t lo = __builtin_amdgcn_perm(p23, p01, 0x0C0C0400u);
+    const uint32_t hi = __builtin_amdgcn_perm(p67, p45, 0x0C0C0400u);
+    return __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+}
+
 // grid = (strips, H): a workgroup owns one strip of one head, both planes;
 // every lane runs two row jobs (key, value), whose loads go out together
 // with the slot loads before the first rotation.
@@ -348,129 +318,406 @@ __global__ __launch_bounds__(kWriterThreads) void strip_writer(
     uint32_t* strip_words =
         (uint32_t*)(value_cache + (head_base + (tip & ~(uint32_t)15)) * (D / 2));
     for (int w = tid; w < D * 2; w += kWriterThreads) {
-        const int channel = w >> 1, half = w & 1;
-        const uint32_t* src = &lds_t[channel >> 3][8 * half];
-        const uint4 a = *(const uint4*)src;
-        const uint4 b = *(const uint4*)(src + 4);
-        const uint32_t sh = 4u * (uint32_t)(channel & 7);
-        const uint32_t n[8] = {__builtin_amdgcn_ubfe(a.x, sh, 4), __builtin_amdgcn_ubfe(a.y, sh, 4),
-                               __builtin_amdgcn_ubfe(a.z, sh, 4), __builtin_amdgcn_ubfe(a.w, sh, 4),
-                               __builtin_amdgcn_ubfe(b.x, sh, 4), __builtin_amdgcn_ubfe(b.y, sh, 4),
-                               __builtin_amdgcn_ubfe(b.z, sh, 4), __builtin_amdgcn_ubfe(b.w, sh, 4)};
-        const uint32_t p01 = (n[1] << 4) | n[0];
-        const uint32_t p23 = (n[3] << 4) | n[2];
-        const uint32_t p45 = (n[5] << 4) | n[4];
-        const uint32_t p67 = (n[7] << 4) | n[6];
-        const uint32_t lo = __builtin_amdgcn_perm(p23, p01, 0x0C0C0400u);
-        const uint32_t hi = __builtin_amdgcn_perm(p67, p45, 0x0C0C0400u);
-        strip_words[w] = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+        strip_words[w] = strip_word(lds_t, w);
     }
 }
 
 // ----------------------------------------------------------- scatter writer
-// One workgroup walks items item_begin + blockIdx.x, += gridDim.x. Inside an
-// item the tokens are grouped into runs of consecutive slots inside one strip
-// (at most 16), exactly the reference's transaction unit.
+// Requests of several tokens (cu_seqlens). The reference walks a (request,
+// head) item's tokens in order, run by run; here a request is cut into
+// chunks of 16 tokens that workgroups take independently, with the same bytes
+// as that walk for any slots:
+//   * Chunk c holds tokens 16c - a .. 16c - a + 15, a the first slot's place
+//     in its strip, so a request written at consecutive positions has one
+//     strip to a chunk, wherever it begins.
+//   * A chunk whose valid tokens sit at consecutive slots of one strip that no
+//     other token of the request touches is written at once (scatter_chunk):
+//     the strip writer's arithmetic and transpose, the value strip's words
+//     merged under the mask of the columns written (whole words are stored
+//     without a read). To know that no other token touches the strip, the
+//     workgroup reads the request's slots (4 bytes a token against the
+//     5 x head_size bytes a head of the token costs) under its rows' loads.
+//   * Any other chunk goes token by token (scatter_tokens): a strip belongs to
+//     the chunk that holds its first token, which writes all of its tokens in
+//     token order; the other chunks skip them. So one workgroup at a time
+//     merges into a strip, and of two tokens with one slot the later wins.
+// A workgroup takes a run of (chunk, head) pairs: the slots are read once for
+// the heads of a chunk, and the next head's rows are in flight under the
+// current head's arithmetic.
+// 8 ragged chunks of 17..2048 tokens (8256 tokens, 8 heads of 128):
+// 790 us a (request, head) item at a time, 18.0 us in chunks; bound there by
+// the vector ALU (about 310 instructions a wave, chunk and head) and by the
+// chain of loads that a chunk begins with (lengths, slots, rows).
+
+// One lane's CPL consecutive BF16 channels as loaded (any alignment).
+template <int CPL>
+struct RawRow {
+    uint32_t w[CPL / 2];
+};
+
+template <int CPL>
+__device__ __forceinline__ void load_raw(const uint16_t* src, RawRow<CPL>& r)
+{
+    __builtin_memcpy(r.w, src, CPL * 2);
+}
+
+template <int CPL>
+__device__ __forceinline__ void unpack_raw(const RawRow<CPL>& r, float (&v)[CPL])
+{
+#pragma unroll
+    for (int i = 0; i < CPL / 2; ++i) {
+        v[2 * i] = __uint_as_float(r.w[i] << 16);
+        v[2 * i + 1] = __uint_as_float(r.w[i] & 0xffff0000u);
+    }
+}
+
+// Exact policy on both rows (held as sigma * v, absmax a): t as the strip
+// writer's (kQMagic + code as bits). Rows with an absmax below 2^-100, zero or
+// infinite (their power of two is not a normal float, or the row has its own
+// rule: zero rows store codes 0 and scale 1, -inf stores code 0) take the
+// written-out form behind a wave vote.
+template <int CPL>
+__device__ __forceinline__ void quantise_exact(const float (&v)[2][CPL], const float (&a)[2],
+                                               float sigma, float inv_sqrt_len,
+                                               uint32_t (&t)[2][CPL], float (&scale)[2])
+{
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        const uint32_t field = __float_as_uint(a[r]) >> 23;  // a >= 0
+        const float p2 = sigma * __uint_as_float((256u - field) << 23);  // 2^(2-e)
+#pragma unroll
+        for (int j = 0; j < CPL; ++j)
+            t[r][j] = __float_as_uint(fminf(__builtin_fmaf(v[r][j], p2, kQMagic), kQMagicTop));
+        scale[r] = __uint_as_float((field - 2u) << 23) * inv_sqrt_len;
+    }
+    const bool odd0 = !(a[0] >= 0x1p-100f && a[0] < INFINITY);
+    const bool odd1 = !(a[1] >= 0x1p-100f && a[1] < INFINITY);
+    if (__builtin_expect(__any(odd0 || odd1), 0)) {
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            if (!(r == 0 ? odd0 : odd1)) continue;
+            const bool zero = a[r] == 0.0f;
+            const int e = zero ? 2 : exponent_of(a[r]);
+#pragma unroll
+            for (int j = 0; j < CPL; ++j) {
+                const float y = fminf(rintf(ldexpf(sigma * v[r][j], 2 - e)), 7.0f);
+                const uint32_t q = zero ? 0u : (uint32_t)(int)y & 0xfu;
+                t[r][j] = 0x4B400000u | (q ^ 8u);
+            }
+            scale[r] = zero ? 1.0f : ldexpf(1.0f, e - 2) * inv_sqrt_len;
+        }
+    }
+}
+
+// The nibble mask of 8 columns (bit i -> nibble i).
+__device__ __forceinline__ uint32_t nibble_mask(uint32_t b)
+{
+    uint32_t x = (b | (b << 12)) & 0x000F000Fu;
+    x = (x | (x << 6)) & 0x03030303u;
+    x = (x | (x << 3)) & 0x11111111u;
+    return x * 15u;
+}
+
+template <int CPL>
+__device__ __forceinline__ void store_key_word(int8_t* dst, const uint32_t (&t)[CPL])
+{
+    if constexpr (CPL == 16)
+        *(uint2*)dst = make_uint2(pack8(t), pack8(&t[8]));
+    else if constexpr (CPL == 8)
+        *(uint32_t*)dst = pack8(t);
+    else
+        *(uint16_t*)dst = (uint16_t)pack4(t);
+}
+
+// Workgroups of the launch: as many as the registers keep resident on 256
+// CUs (four waves a SIMD, three at d = 256), so one generation takes it all.
+// 8 requests of 17..2048 tokens: 512 / 768 / 1024 / 2048 workgroups 18.7 /
+// 17.6 / 18.2 / 20.2 us; one of 8000 tokens 17.4 / 20.1 / 16.2 / 20.2 us.
 template <int D>
-__global__ __launch_bounds__(kWriterThreads) void scatter_writer(
-    const uint16_t* __restrict__ key, const uint16_t* __restrict__ value,
-    int8_t* __restrict__ key_cache, int8_t* __restrict__ value_cache,
-    float* __restrict__ scale_cache, const int32_t* __restrict__ slots,
-    const float* __restrict__ pi_signs, const int32_t* __restrict__ cu_seqlens,
-    int32_t* __restrict__ probe, uint32_t num_requests, uint32_t H, uint32_t S, uint32_t P,
-    uint32_t item_begin, uint32_t item_count, float inv_sqrt_len)
+constexpr uint32_t kScatterGrid = D == 256 ? 768 : 1024;
+constexpr uint32_t kScatterPlan = 1024;  // requests whose chunk prefix is staged on chip
+
+struct ScatterArgs {
+    const uint16_t *key, *value;
+    int8_t *key_cache, *value_cache;
+    float* scale_cache;
+    const int32_t* slots;
+    uint32_t H, S, P;
+    float inv_sqrt_len;
+};
+
+__device__ __forceinline__ bool slot_in_pool(int32_t slot, uint32_t S, uint32_t P)
+{
+    return slot >= 0 && (uint64_t)(uint32_t)slot < (uint64_t)S * P;
+}
+
+// Tokens first .. first + 15 (of the request's n at t0) one at a time, heads
+// [h0, h1): each strip whose first token of the request lies here, with all
+// of its tokens in token order. Every thread of the workgroup runs it (it has
+// barriers); a 16-lane group takes a head, so one lane makes all merges of a
+// strip word, in order.
+template <int D>
+__device__ __forceinline__ void scatter_tokens(const ScatterArgs& p, uint32_t t0, uint32_t n,
+                                               int64_t first, uint32_t h0, uint32_t h1,
+                                               const float (&sign)[D / 16])
 {
     constexpr int CPL = D / 16;
-    __shared__ uint32_t lds_codes[D * kStrip / 4];
     const int tid = threadIdx.x;
-    const int row = tid >> 4;
-    const int lane_in_row = tid & 15;
-
-    if (probe != nullptr && blockIdx.x == 0 && tid < 32) {
-        const int32_t fields[4] = {0, (int32_t)gridDim.x, 1, (int32_t)item_count};
-        probe[tid] = fields[tid >> 3];
-    }
-
-    float sign[CPL];
-    load_signs<CPL>(pi_signs, nullptr, 0, lane_in_row * CPL, sign);
-    const uint64_t item_end = (uint64_t)item_begin + item_count;
-
-    for (uint64_t item = (uint64_t)item_begin + blockIdx.x; item < item_end; item += gridDim.x) {
-        const uint32_t request = (uint32_t)(item / H);
-        const uint32_t head = (uint32_t)(item % H);
-        if (request >= num_requests) continue;
-        uint32_t token = cu_seqlens ? (uint32_t)cu_seqlens[request] : request;
-        const uint32_t token_end = cu_seqlens ? (uint32_t)cu_seqlens[request + 1] : request + 1;
-
-        while (token < token_end) {
-            // Run discovery, computed identically by every lane (uniform).
-            const int32_t slot0 = slots[token];
-            if (slot0 < 0 || (uint32_t)slot0 / S >= P) {
-                ++token;
-                continue;
-            }
-            const uint32_t page = (uint32_t)slot0 / S;
-            const uint32_t tip0 = (uint32_t)slot0 % S;
-            const uint32_t strip_in_page = tip0 / kStrip;
-            uint32_t run = 1;
-            while (token + run < token_end && run < (uint32_t)kStrip) {
-                const int32_t next = slots[token + run];
-                if (next != slot0 + (int32_t)run) break;
-                if ((uint32_t)next / S != page || ((uint32_t)next % S) / kStrip != strip_in_page) break;
-                ++run;
-            }
-            const bool live = (uint32_t)row < run;
-            const uint32_t tok = token + (live ? (uint32_t)row : 0u);
-            const size_t head_base = ((size_t)page * H + head) * S;
-
-            for (uint32_t plane = 0; plane < 2; ++plane) {
-                const uint16_t* src = (plane == 0 ? key : value) +
-                                      ((size_t)tok * H + head) * D + lane_in_row * CPL;
-                float v[CPL];
-                load_row<CPL>(src, v);
-                int q[CPL];
-                const float scale =
-                    rotate_quantise<D, CPL>(v, sign, lane_in_row, inv_sqrt_len, kPolicyExact, q);
-                const uint32_t tip = tip0 + (uint32_t)row;
-                if (live && lane_in_row == 0)
-                    scale_cache[(((size_t)plane * P + page) * H + head) * S + tip] = scale;
-                if (plane == 0) {
-                    if (live)
-                        store_key_codes<CPL>(
-                            key_cache + (head_base + tip) * (D / 2) + lane_in_row * (CPL / 2), q);
-                    continue;
-                }
-                // Value plane: codes to LDS at their strip column, then merge
-                // only the owned nibbles into the words they live in.
-                uint8_t* lds = (uint8_t*)lds_codes;
-                const uint32_t col = (tip0 % kStrip) + (uint32_t)row;
-                if (live) {
+    const int l = row_lane(tid & 15);
+    const float sigma = row_sigma(l);
+    for (int i = 0; i < kStrip; ++i) {
+        const int64_t at = first + i;
+        if (at < 0 || at >= (int64_t)n) continue;
+        const uint32_t i0 = (uint32_t)at;
+        const int32_t slot0 = p.slots[t0 + i0];
+        if (!slot_in_pool(slot0, p.S, p.P)) continue;
+        const int32_t strip = slot0 >> 4;
+        int seen = 0;  // an earlier token of the request in this strip
+        for (uint32_t u = tid; u < i0; u += kWriterThreads) seen |= (p.slots[t0 + u] >> 4) == strip;
+        if (__syncthreads_or(seen)) continue;
+        for (uint32_t base = i0; base < n; base += 64) {
+            const uint32_t u = base + (tid & 63);
+            const bool in = u < n && (p.slots[t0 + u] >> 4) == strip;
+            for (uint64_t m = __ballot(in); m != 0; m &= m - 1) {
+                const uint32_t token = t0 + base + (uint32_t)__builtin_ctzll(m);
+                const uint32_t slot = (uint32_t)p.slots[token];
+                const uint32_t page = slot / p.S, tip = slot % p.S, col = tip % kStrip;
+                for (uint32_t h = h0 + (tid >> 4); h < h1; h += kWriterThreads / 16) {
+                    const size_t src = ((size_t)token * p.H + h) * D + l * CPL;
+                    RawRow<CPL> rk, rv;
+                    load_raw<CPL>(p.key + src, rk);
+                    load_raw<CPL>(p.value + src, rv);
+                    float v[2][CPL], a[2], sc[2];
+                    unpack_raw<CPL>(rk, v[0]);
+                    unpack_raw<CPL>(rv, v[1]);
+                    writer_rotate<D, CPL>(v, sign, l);
+                    writer_absmax<CPL>(v, 0.0f, a);
+                    uint32_t t[2][CPL];
+                    quantise_exact<CPL>(v, a, sigma, p.inv_sqrt_len, t, sc);
+                    const size_t row = ((size_t)page * p.H + h) * p.S + tip;
+                    if ((tid & 15) == 0) {
+                        p.scale_cache[row] = sc[0];
+                        p.scale_cache[(size_t)p.P * p.H * p.S + row] = sc[1];
+                    }
+                    store_key_word<CPL>(p.key_cache + row * (D / 2) + l * (CPL / 2), t[0]);
+                    uint32_t* words = (uint32_t*)(p.value_cache + (row - col) * (D / 2)) +
+                                      2 * l * CPL + (col >> 3);
+                    const uint32_t sh = 4u * (col & 7u);
 #pragma unroll
                     for (int j = 0; j < CPL; ++j)
-                        lds[(lane_in_row * CPL + j) * kStrip + col] = (uint8_t)(q[j] & 0xf);
+                        words[2 * j] = (words[2 * j] & ~(0xfu << sh)) |
+                                       (((t[1][j] ^ 8u) & 0xfu) << sh);
                 }
-                __syncthreads();
-                const uint32_t first = tip0 % kStrip, last = first + run;  // owned columns
-                uint32_t* strip_words =
-                    (uint32_t*)(value_cache + (head_base + strip_in_page * kStrip) * (D / 2));
-                for (int w = tid; w < D * 2; w += kWriterThreads) {
-                    const int channel = w >> 1, half = w & 1;
-                    const uint32_t t0 = (uint32_t)half * 8u;
-                    const uint32_t lo = first > t0 ? first : t0;
-                    const uint32_t hi = last < t0 + 8u ? last : t0 + 8u;
-                    if (lo >= hi) continue;
-                    uint32_t mask = 0u, bits = 0u;
-                    for (uint32_t t = lo; t < hi; ++t) {
-                        const uint32_t sh = 4u * (t - t0);
-                        mask |= 0xfu << sh;
-                        bits |= (uint32_t)lds[channel * kStrip + t] << sh;
-                    }
-                    strip_words[w] = (strip_words[w] & ~mask) | bits;
-                }
-                __syncthreads();
             }
-            token += run;
         }
+    }
+}
+
+// One chunk of 16 tokens (first .. first + 15 of the request's n at t0), heads
+// [h0, h1). False: nothing is written, the chunk goes token by token.
+template <int D>
+__device__ __forceinline__ bool scatter_chunk(const ScatterArgs& p, uint32_t t0, uint32_t n,
+                                              int64_t first, uint32_t h0, uint32_t h1,
+                                              const float (&sign)[D / 16],
+                                              uint32_t (*lds_t)[D / 8][20], int* clash_w)
+{
+    constexpr int CPL = D / 16;
+    const int tid = threadIdx.x;
+    const int row = tid >> 4;
+    const int l = row_lane(tid & 15);
+    const float sigma = row_sigma(l);
+
+    // the first head's rows, and lane j of every 16 the slot of token j
+    const int64_t at = first + row;
+    const uint32_t tok = t0 + (uint32_t)(at < 0 ? 0 : at < (int64_t)n ? at : (int64_t)n - 1);
+    const size_t src0 = ((size_t)tok * p.H + h0) * D + l * CPL;
+    RawRow<CPL> rk, rv;
+    load_raw<CPL>(p.key + src0, rk);
+    load_raw<CPL>(p.value + src0, rv);
+    const int j16 = tid & 15;
+    const int64_t aj = first + j16;
+    const int32_t slot_j = aj >= 0 && aj < (int64_t)n ? p.slots[t0 + (uint32_t)aj] : -1;
+    const bool valid_j = slot_in_pool(slot_j, p.S, p.P);
+    const uint32_t vmask = (uint32_t)__ballot(valid_j) & 0xffffu;  // the same in every wave
+    if (vmask == 0) return true;
+    // regular: every valid token j at slot base + j, all in one strip
+    const int lead = __builtin_ctz(vmask);
+    const int32_t base = __builtin_amdgcn_readlane(slot_j, lead) - lead;
+    const int32_t strip = (base + lead) >> 4;
+    const bool odd = valid_j && (slot_j - j16 != base || (slot_j >> 4) != strip);
+    const bool regular = __ballot(odd) == 0;
+    // does another token of the request touch the strip?
+    int clash = !regular;
+    if (regular) {
+        // eight loads in flight a thread (past the end: the last token again)
+        const int32_t* sl = p.slots + t0;
+        const uint32_t f = (uint32_t)first;  // mod 2^32, as the distance below
+        for (uint32_t u0 = tid; u0 < n; u0 += 8 * kWriterThreads) {
+            int32_t s[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) s[k] = sl[min(u0 + k * kWriterThreads, n - 1)];
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                clash |= (s[k] >> 4) == strip &&
+                         min(u0 + k * kWriterThreads, n - 1) - f >= (uint32_t)kStrip;
+        }
+    }
+    const int wc = __any(clash);
+    if ((tid & 63) == 0) clash_w[tid >> 6] = wc;
+
+    const int shift = base - strip * kStrip;           // column of token j: j + shift
+    const uint32_t cmask = shift >= 0 ? vmask << shift : vmask >> -shift;  // columns written
+    const uint32_t m0 = nibble_mask(cmask & 0xffu), m1 = nibble_mask((cmask >> 8) & 0xffu);
+    const bool whole = (cmask & 0xffffu) == 0xffffu;
+    const uint32_t page = (uint32_t)(base + lead) / p.S;
+    const uint32_t strip_tip = (uint32_t)strip * kStrip - page * p.S;
+    const bool mine = (vmask >> row) & 1u;
+    const uint32_t col = (uint32_t)(row + shift) & 15u;
+    const size_t plane = (size_t)p.P * p.H * p.S;
+    constexpr int NW = (2 * D + kWriterThreads - 1) / kWriterThreads;  // strip words a thread
+
+    for (uint32_t h = h0, it = 0; h < h1; ++h, ++it) {
+        const size_t srow = ((size_t)page * p.H + h) * p.S + strip_tip;  // the strip's first row
+        uint32_t* words = (uint32_t*)(p.value_cache + srow * (D / 2));
+        float v[2][CPL];
+        unpack_raw<CPL>(rk, v[0]);
+        unpack_raw<CPL>(rv, v[1]);
+        if (h + 1 < h1) {
+            const size_t src = src0 + (size_t)(it + 1) * D;
+            load_raw<CPL>(p.key + src, rk);
+            load_raw<CPL>(p.value + src, rv);
+        }
+        uint32_t old[NW];
+        if (!whole) {
+#pragma unroll
+            for (int k = 0; k < NW; ++k)
+                old[k] = tid + k * kWriterThreads < 2 * D ? words[tid + k * kWriterThreads] : 0u;
+        }
+        writer_rotate<D, CPL>(v, sign, l);
+        float a[2], sc[2];
+        writer_absmax<CPL>(v, 0.0f, a);
+        uint32_t t[2][CPL];
+        quantise_exact<CPL>(v, a, sigma, p.inv_sqrt_len, t, sc);
+        uint32_t(*buf)[20] = lds_t[it & 1];
+        if (mine) {
+            if constexpr (CPL >= 8) {
+#pragma unroll
+                for (int k = 0; k < CPL / 8; ++k) buf[l * (CPL / 8) + k][col] = pack8(&t[1][8 * k]);
+            } else {
+                ((uint16_t*)&buf[l >> 1][col])[l & 1] = (uint16_t)pack4(t[1]);
+            }
+        }
+        // one barrier a head: the buffer written two heads on is read before
+        // the barrier in between
+        lds_barrier();
+        if (it == 0) {
+            const int4 c4 = *(const int4*)clash_w;
+            if (c4.x | c4.y | c4.z | c4.w) return false;
+        }
+        if (mine) {
+            const size_t r = srow + col;
+            if ((tid & 15) == 0) {
+                p.scale_cache[r] = sc[0];
+                p.scale_cache[plane + r] = sc[1];
+            }
+            store_key_word<CPL>(p.key_cache + r * (D / 2) + l * (CPL / 2), t[0]);
+        }
+#pragma unroll
+        for (int k = 0; k < NW; ++k) {
+            const int w = tid + k * kWriterThreads;
+            const uint32_t m = (w & 1) ? m1 : m0;
+            if (w < 2 * D && m != 0) {
+                const uint32_t bits = strip_word(buf, w);
+                words[w] = whole ? bits : (old[k] & ~m) | (bits & m);
+            }
+        }
+    }
+    return true;
+}
+
+// The lengths are on the device only, so the grid is fixed: every workgroup
+// counts the requests' chunks (a prefix over the requests of the window,
+// staged in LDS; a request of n tokens has at most (n + 30) / 16 chunks) and
+// takes an equal run of the (chunk, head) pairs.
+template <int D>
+__global__ __launch_bounds__(kWriterThreads, D == 256 ? 3 : 4) void scatter_writer(
+    ScatterArgs p, const float* __restrict__ pi_signs, const int32_t* __restrict__ cu_seqlens,
+    int32_t* __restrict__ probe, uint32_t probe_grid, uint32_t num_requests, uint32_t item_begin,
+    uint32_t item_count)
+{
+    constexpr int CPL = D / 16;
+    __shared__ __align__(16) uint32_t lds_t[2][D / 8][20];
+    __shared__ __align__(16) int clash_w[kWriterThreads / 64];
+    __shared__ uint32_t chunks[kScatterPlan];  // inclusive prefix of the requests' chunks
+    const int tid = threadIdx.x, lane = tid & 63;
+
+    if (probe != nullptr && blockIdx.x == 0 && tid < 32) {
+        const int32_t fields[4] = {0, (int32_t)probe_grid, 1, (int32_t)item_count};
+        probe[tid] = fields[tid >> 3];
+    }
+    const uint64_t item_end = (uint64_t)item_begin + item_count;
+    const uint32_t r0 = item_begin / p.H;
+    const uint32_t r1 = (uint32_t)min((uint64_t)num_requests, (item_end + p.H - 1) / p.H);
+    if (r1 <= r0) return;
+    float sign[CPL];
+    load_signs<CPL>(pi_signs, nullptr, 0, row_lane(tid & 15) * CPL, sign);
+
+    for (uint64_t rb = r0; rb < r1; rb += kScatterPlan) {
+        const uint32_t nr = (uint32_t)min((uint64_t)kScatterPlan, r1 - rb);
+        const int32_t* cu = cu_seqlens + rb;
+        if (tid < 64) {
+            uint32_t carry = 0;
+            for (uint32_t b = 0; b < nr; b += 64) {
+                const uint32_t i = min(b + lane, nr - 1);
+                const uint32_t t0 = (uint32_t)cu[i], t1 = (uint32_t)cu[i + 1];
+                uint32_t v = b + lane < nr && t1 > t0 ? (t1 - t0 + 30u) >> 4 : 0u;
+#pragma unroll
+                for (int o = 1; o < 64; o <<= 1) {
+                    const uint32_t w = __shfl_up(v, o, 64);
+                    if (lane >= o) v += w;
+                }
+                v += carry;
+                if (b + lane < nr) chunks[i] = v;
+                carry = __shfl(v, 63, 64);
+            }
+        }
+        lds_barrier();
+        // an equal run of (chunk, head) pairs to every workgroup
+        const uint32_t total = __builtin_amdgcn_readfirstlane(chunks[nr - 1]);
+        const uint64_t pairs = (uint64_t)total * p.H;
+        const uint64_t per = (pairs + kScatterGrid<D> - 1) / kScatterGrid<D>;
+        const uint64_t at = per * blockIdx.x;
+        uint32_t v = pairs <= 0xffffffffull ? (uint32_t)at / p.H : (uint32_t)(at / p.H);
+        uint32_t h = (uint32_t)(at - (uint64_t)v * p.H);
+        uint32_t i = nr;  // the first request whose prefix passes v
+        for (uint32_t b = 0; b < nr && at < pairs; b += 64) {
+            const uint64_t m = __ballot(b + lane < nr && chunks[b + lane] > v);
+            if (m != 0) {
+                i = b + (uint32_t)__builtin_ctzll(m);
+                break;
+            }
+        }
+        i = __builtin_amdgcn_readfirstlane(i);
+        for (uint64_t left = per; left > 0 && i < nr;) {
+            const uint32_t take = (uint32_t)min(left, (uint64_t)(p.H - h));
+            const uint32_t c = v - (i > 0 ? chunks[i - 1] : 0u);
+            const uint64_t item0 = (rb + i) * p.H;  // the request's heads inside the window
+            const uint32_t h0 = (uint32_t)(max(item0 + h, (uint64_t)item_begin) - item0);
+            const uint32_t h1 = (uint32_t)(min(item0 + h + take, item_end) - item0);
+            const uint32_t t0 = (uint32_t)cu[i], n = (uint32_t)cu[i + 1] - t0;
+            const int32_t s0 = p.slots[t0];
+            const int64_t first = (int64_t)c * kStrip - (s0 >= 0 ? s0 % kStrip : 0);
+            if ((int32_t)(h1 - h0) > 0 && first < (int64_t)n) {
+                if (!scatter_chunk<D>(p, t0, n, first, h0, h1, sign, lds_t, clash_w))
+                    scatter_tokens<D>(p, t0, n, first, h0, h1, sign);
+            }
+            lds_barrier();  // the next chunk writes clash_w and the first buffer again
+            left -= take;
+            h = 0;
+            ++v;
+            while (i < nr && __builtin_amdgcn_readfirstlane(chunks[i]) <= v) ++i;
+        }
+        lds_barrier();
     }
 }
 
@@ -656,6 +903,8 @@ hipError_t launch_scatter_writer(hipStream_t stream, uint32_t grid, const uint16
     // launch probe reports
     const uint64_t groups = ((uint64_t)item_count + 15) / 16;
     const uint32_t tgrid = (uint32_t)(groups < 4096 ? groups : 4096);
+    const ScatterArgs args{key, value, key_cache, value_cache, scale_cache, slots, H, S, P,
+                           inv_sqrt_len};
 #define TQ4_SCATTER_CASE(DD)                                                                      \
     if (D == DD) {                                                                                \
         if (cu_seqlens == nullptr)                                                                \
@@ -664,10 +913,9 @@ hipError_t launch_scatter_writer(hipStream_t stream, uint32_t grid, const uint16
                                pi_signs, probe, grid, num_requests, H, S, P, item_begin,          \
                                item_count, inv_sqrt_len);                                         \
         else                                                                                      \
-            hipLaunchKernelGGL((scatter_writer<DD>), dim3(grid), dim3(kWriterThreads), 0, stream, \
-                               key, value, key_cache, value_cache, scale_cache, slots, pi_signs,  \
-                               cu_seqlens, probe, num_requests, H, S, P, item_begin, item_count,  \
-                               inv_sqrt_len);                                                     \
+            hipLaunchKernelGGL((scatter_writer<DD>), dim3(kScatterGrid<DD>), dim3(kWriterThreads), 0, \
+                               stream, args, pi_signs, cu_seqlens, probe, grid, num_requests,     \
+                               item_begin, item_count);                                           \
         return hipGetLastError();                                                                 \
     }
     TQ4_SCATTER_CASE(64)

@@ -109,9 +109,10 @@ int tq4_reshape_and_cache_bf16(void* stream, const uint16_t* key, const uint16_t
  * The value strip is read-modify-written nibble-exactly: every nibble the
  * launch does not own is preserved. Quantiser: exact absmax, absmax == 0
  * gives codes 0 and scale 1.0 (turboquant_scatter_oracle.hpp:185-217).
- * block_dim is a grid-size hint (0 = one workgroup per item). When
- * launch_probe is non-NULL, workgroup 0 writes int32[32]: lanes 0-7 its
- * block index, 8-15 the grid size, 16-23 1, 24-31 item_count.
+ * block_dim is a grid-size hint (0 = one workgroup per item) that the probe
+ * reports; the grid is chosen here. When launch_probe is non-NULL, workgroup
+ * 0 writes int32[32]: lanes 0-7 its block index, 8-15 the grid size, 16-23 1,
+ * 24-31 item_count.
  * Two work items of one launch must not own tokens of the same strip.
  * Replaces launch_turboquant_reshape_scatter_aiv
  * (kernels/ops/turboquant/turboquant_reshape_scatter_aiv.cpp:760-773).
