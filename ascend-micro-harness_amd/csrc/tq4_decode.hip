@@ -915,8 +915,11 @@ __device__ __forceinline__ void finish_item(const DecodeParams& p, uint32_t seq,
                 const float vv[4] = {v.x, v.y, v.z, v.w};
                 rec_store<4, true>(rsrc, r * row_bytes + (4 + ch) * 4u, vv);
                 if (ch == 0) {
-                    const float h[4] = {M == -INFINITY ? kMasked : M * kLn2, L, 0.0f, 0.0f};
-                    rec_store<4, true>(rsrc, r * row_bytes, h);
+                    // (m, l) only: the combiner clears what it reads, and a
+                    // padding word left behind would read as a written word
+                    // under another split count's record layout
+                    const float h[2] = {M == -INFINITY ? kMasked : M * kLn2, L};
+                    rec_store<2, true>(rsrc, r * row_bytes, h);
                 }
             }
             TQ4_STAMP(6, TQ4_NOW);

@@ -565,3 +565,33 @@ def test_persistent_repeat_and_graph(tq4, oracle):
         assert np.array_equal(host(out), first)
         call()
         assert np.array_equal(host(out), first)
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("K", [2, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("B", [2, 160])
+def test_record_chunk_edges(tq4, oracle, d, K, B):
+    """Split counts at the edges of the combiner's record chunks (4, 8 and 16
+    splits), sequences with fewer live splits among them, a full and a partial
+    GQA group, the one-launch and the persistent kernel; the zeroed workspace
+    of one split count serves the next."""
+    import torch
+    rng = np.random.default_rng(1000 * d + 10 * K + B)
+    G, H, S = (16, 2, 16) if B == 2 else (3, 4, 16)
+    ctx = [int(x) for x in rng.integers(1, 16 * K + 1, B)]
+    ctx[0] = 16 * K  # a page to a split, every split live
+    P = sum((c + 15) // 16 for c in ctx) + 8
+    kc, vc, sc, tables, signs, isl = build_cache(oracle, rng, ctx, H, d, S, P)
+    q = f32_to_bf16(rng.standard_normal((B, G * H, d)).astype(np.float32))
+    scale = np.float32(1.0 / math.sqrt(d))
+    ctx_a = np.array(ctx, np.int32)
+    _, want = oracle.paged_decode(q, kc, vc, sc, tables, ctx_a, signs, None, G * H, H, d, S, P, K,
+                                  scale, isl, 1, threads=8)
+    ws = tq4.decode_workspace(B, G * H, H, d, 16)
+    args = [dev(q), dev(kc), dev(vc), dev(sc), dev(tables), dev(ctx_a), dev(signs)]
+    outs = [host(tq4.paged_decode(*args, H, S, P, workspace=ws, num_splits=k, scale=float(scale),
+                                  inv_sqrt_len=float(isl))) for k in (K, 3, K)]
+    check_out(outs[0], want, f"record chunks d {d} K {K} B {B}")
+    assert np.array_equal(outs[0], outs[2])
+    assert tq4.decode_poll_timeouts(ws, B, H) == 0
+    assert not torch.any(ws)
