@@ -797,7 +797,7 @@ __device__ __forceinline__ void park_rows(const RowState<D>& st, bool row_live, 
 // the partial record; MODE 1 takes the split's place in the fused combine
 // (export, or finalise from LDS when it is the only live split, or combine as
 // the last ticket). region: the item's q staging / merge region.
-template <int D, int MODE, bool OWN>
+template <int D, int MODE, bool OWN, int NS>
 __device__ __forceinline__ void finish_item(const DecodeParams& p, uint32_t seq, uint32_t kvh,
                                             uint32_t split, uint32_t k_live, uint32_t ticket,
                                             const RowState<D>& st, bool row_live, float* region)
@@ -960,13 +960,13 @@ __device__ __forceinline__ void finish_item(const DecodeParams& p, uint32_t seq,
                 };
                 auto none = [](uint32_t(&)[2], uint32_t(&)[CC]) {};
                 float v[CC];
-                // 16 splits per chunk: wider chunks (32 per round trip)
-                // measured slower at every split count from 17 to 64
+                // 2 * NS splits per chunk, 16 at most: wider chunks (32 per
+                // round trip) measured slower at every split count from 17 to 64
                 if constexpr (OWN)
-                    combine_records<D, true, 8>(p.records + qh * p.K * RS, k_live, lane, v,
+                    combine_records<D, true, NS>(p.records + qh * p.K * RS, k_live, lane, v,
                                                 split, own, p.poll_limit, p.timeouts);
                 else
-                    combine_records<D, true, 8>(p.records + qh * p.K * RS, k_live, lane, v, ~0u,
+                    combine_records<D, true, NS>(p.records + qh * p.K * RS, k_live, lane, v, ~0u,
                                                 none, p.poll_limit, p.timeouts);
                 if (g == 0) TQ4_STAMP(7, TQ4_NOW);
                 egress_row<D>(v, es, gt, p.out + qh * D, p.inv_sqrt_len, p.output_stage, lane);
@@ -1008,7 +1008,7 @@ struct NoHook {
     __device__ void operator()() const {}
 };
 
-template <int D, int MODE, bool OWN = true, class Hook = NoHook>
+template <int D, int MODE, int NS, bool OWN = true, class Hook = NoHook>
 __device__ __forceinline__ void decode_item(const DecodeParams& p, const uint32_t seq,
                                             const uint32_t kvh, const uint32_t split,
                                             Hook&& after_issue = Hook())
@@ -1277,7 +1277,7 @@ __device__ __forceinline__ void decode_item(const DecodeParams& p, const uint32_
     }
 
     TQ4_STAMP(4, TQ4_NOW);
-    finish_item<D, MODE, OWN>(p, seq, kvh, split, k_live, ticket, st, qo.row_live, region);
+    finish_item<D, MODE, OWN, NS>(p, seq, kvh, split, k_live, ticket, st, qo.row_live, region);
 }
 
 // Waves per SIMD the register ring allows without spilling: two at d = 64
@@ -1287,11 +1287,11 @@ __device__ __forceinline__ void decode_item(const DecodeParams& p, const uint32_
     __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2, 2)))
 
 // One workgroup per (seq, kv head, split), splits fastest.
-template <int D, int MODE>
+template <int D, int MODE, int NS>
 __global__ TQ4_DECODE_ATTRS void decode_kernel(DecodeParams p)
 {
     const uint32_t item = blockIdx.x;
-    decode_item<D, MODE>(p, item / (p.K * p.Hkv), (item / p.K) % p.Hkv, item % p.K);
+    decode_item<D, MODE, NS>(p, item / (p.K * p.Hkv), (item / p.K) % p.Hkv, item % p.K);
 }
 
 // Persistent fused decode for launches with more work items than
@@ -1440,7 +1440,7 @@ __device__ __forceinline__ void item_coords(const DecodeParams& p, uint32_t item
     }
 }
 
-template <int D>
+template <int D, int NS>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2, 2)))
 void decode_persistent_kernel(DecodeParams p)
 {
@@ -1475,7 +1475,7 @@ void decode_persistent_kernel(DecodeParams p)
         TQ4_STAMP_P(13, split);
         // the next item's queue fetch goes out after this item's first strip
         // loads (decode_item's hook); its value is read after the item
-        decode_item<D, 1, false>(p, seq, kvh, split, [&]() {
+        decode_item<D, 1, NS, false>(p, seq, kvh, split, [&]() {
             if (tid == 0)
                 fetched = __hip_atomic_fetch_add(subq, 1u, __ATOMIC_RELAXED,
                                                  __HIP_MEMORY_SCOPE_AGENT);
@@ -1542,29 +1542,46 @@ uint32_t persistent_slots(Kernel kernel, size_t lds)
     return cus > 0 && per_cu > 0 ? (uint32_t)cus * (uint32_t)per_cu : 0u;
 }
 
+// The fused decode with record chunks of 2 * NS splits.
+template <int D, int NS>
+hipError_t launch_fused_t(hipStream_t stream, const DecodeParams& p, size_t lds)
+{
+    const size_t blocks = (size_t)p.B * p.Hkv * p.K;
+    // Persistent when the split grid outnumbers the resident slots.
+    if (p.queue != nullptr && p.K > 1 && p.B <= kPersistentMaxSeqs) {
+        const size_t lds_p = lds + (p.B <= kLptMaxSeqs ? 3 : 2) * (size_t)p.B * sizeof(uint32_t);
+        const uint32_t slots = persistent_slots(decode_persistent_kernel<D, NS>, lds_p);
+        if (slots > 0 && blocks > slots) {
+            hipLaunchKernelGGL((decode_persistent_kernel<D, NS>), dim3(slots), dim3(kThreads),
+                               lds_p, stream, p);
+            return hipGetLastError();
+        }
+    }
+    hipLaunchKernelGGL((decode_kernel<D, 1, NS>), dim3((uint32_t)blocks), dim3(kThreads), lds,
+                       stream, p);
+    return hipGetLastError();
+}
+
 template <int D>
 hipError_t launch_decode_t(hipStream_t stream, const DecodeParams& p, int mode)
 {
     const size_t blocks = (size_t)p.B * p.Hkv * p.K;
     const size_t lds = (kHdrFloats + kStripSlots + region_floats(p.G, D)) * sizeof(float);
     if (mode == 0) {
-        hipLaunchKernelGGL((decode_kernel<D, 0>), dim3((uint32_t)blocks), dim3(kThreads), lds,
+        hipLaunchKernelGGL((decode_kernel<D, 0, 8>), dim3((uint32_t)blocks), dim3(kThreads), lds,
                            stream, p);
         return hipGetLastError();
     }
-    // Fused: persistent when the split grid outnumbers the resident slots.
-    if (p.queue != nullptr && p.K > 1 && p.B <= kPersistentMaxSeqs) {
-        const size_t lds_p = lds + (p.B <= kLptMaxSeqs ? 3 : 2) * (size_t)p.B * sizeof(uint32_t);
-        const uint32_t slots = persistent_slots(decode_persistent_kernel<D>, lds_p);
-        if (slots > 0 && blocks > slots) {
-            hipLaunchKernelGGL((decode_persistent_kernel<D>), dim3(slots), dim3(kThreads), lds_p,
-                               stream, p);
-            return hipGetLastError();
-        }
-    }
-    hipLaunchKernelGGL((decode_kernel<D, 1>), dim3((uint32_t)blocks), dim3(kThreads), lds, stream,
-                       p);
-    return hipGetLastError();
+    // The combiner loads, checks and zeroes whole chunks (slots past the live
+    // splits repeat the last one), so few splits take a small chunk. Chosen
+    // by the launch's split count: chosen in the kernel by the live splits, it
+    // cost the 16-split launch 0.3 us. Chunks of 16 / of the smallest of 4, 8
+    // and 16 that holds K: 4 sequences x 8 kv heads, ctx 2048 (K = 8) 8.3 /
+    // 7.6 us; 8 x 8, ctx 300..3000 (K = 4) 10.7 / 9.5 us; 64 x 8, ctx
+    // 512..8192 (K = 3) 68.4 / 66.9 us.
+    if (p.K <= 4) return launch_fused_t<D, 2>(stream, p, lds);
+    if (p.K <= 8) return launch_fused_t<D, 4>(stream, p, lds);
+    return launch_fused_t<D, 8>(stream, p, lds);
 }
 
 template <int D>
