@@ -16,14 +16,13 @@
 //                tests/npu/bench/bench_turboquant_reshape_and_cache.cpp:55-61
 //
 // MI355X design: a vector is spread over 16 lanes of one wave row, d/16
-// consecutive channels per lane (one 16-byte load of BF16 at d = 128), 16
-// vectors per 256-lane workgroup, in the row lane order of the TQ4 writers
-// (row_lane). The FWHT runs in registers below d/16 and as DPP-fed fused
-// butterflies above (row_fmac_stage, same a+b / a-b bits); the sum of
-// squares is a sequential per-lane sum and a 4-step tree over logical lanes. The level needs no table walk: since t_{14-i} = -t_i and
-// t_7 = 0, a positive z counts 8 + #{t_8..t_14 < z} and a negative one
-// 7 - #{t_8..t_14 <= -z}, each a 3-step binary search over seven constants.
-// A row's d/2 packed bytes leave as one coalesced run (d/32 bytes per lane).
+// consecutive channels per lane (one 16-byte load of BF16 at d = 128), in the
+// row lane order of the TQ4 writers (row_lane). The FWHT runs in registers
+// below d/16 and as DPP-fed fused butterflies above (row_fmac_stage, same a+b
+// / a-b bits); the sum of squares is a sequential per-lane sum and a 4-step
+// tree over logical lanes. The level is one comparison: bins a quarter wide
+// hold at most one threshold each (level_of). A row's d/2 packed bytes leave
+// as one coalesced run (d/32 bytes per lane).
 // Built with -ffp-contract=off: every FP32 operation is the one written, so the
 // bits are those of the C oracle's restatement.
 #include <hip/hip_runtime.h>
@@ -71,159 +70,176 @@ __device__ __forceinline__ float sqrt_rn(float x)
     return tiny ? s * 0x1.0p-16f : s;
 }
 
-// The level search by bins of |z| a quarter wide: bin b < 10 is [b/4,
-// (b+1)/4), bin 10 is [2.5, inf]. The positive thresholds lie more than a
-// quarter apart and none on a multiple of a quarter, so a bin holds at most
-// one of them: #{k : kPos[k] < a} = below + (inside < a) of a's bin, `below`
-// counting the thresholds under the bin and `inside` its own (+inf when it
-// has none). 4a and its truncation are exact, so the count is.
+// The level search by bins a quarter wide over the signed line: bin 0 is below
+// -2.5, bin i = 1 .. 20 is [(i - 11)/4, (i - 10)/4), bin 21 is [2.5, inf]. The
+// 15 thresholds lie more than a quarter apart and, but for t_7 = 0 (the first
+// point of its bin), away from the bins' ends, so a bin holds at most one:
+// #{i : t_i < z} = below + (inside < z) of z's bin, `below` counting the
+// thresholds under the bin and `inside` its own (+inf when it has none).
 struct LevelBin {
     float inside;
     uint32_t below;
 };
-constexpr int kLevelBins = 11;
+constexpr int kLevelBins = 22;
+constexpr float kInf = __builtin_inff();
 constexpr LevelBin kBins[kLevelBins] = {
-    {__builtin_inff(), 0}, {kPos[0], 0}, {kPos[1], 1}, {kPos[2], 2}, {kPos[3], 3},
-    {kPos[4], 4},          {__builtin_inff(), 5}, {kPos[5], 5}, {__builtin_inff(), 6},
-    {kPos[6], 6},          {__builtin_inff(), 7}};
+    {kInf, 0},     {-kPos[6], 0}, {kInf, 1},     {-kPos[5], 1}, {kInf, 2},     {-kPos[4], 2},
+    {-kPos[3], 3}, {-kPos[2], 4}, {-kPos[1], 5}, {-kPos[0], 6}, {kInf, 7},     {0.0f, 7},
+    {kPos[0], 8},  {kPos[1], 9},  {kPos[2], 10}, {kPos[3], 11}, {kPos[4], 12}, {kInf, 13},
+    {kPos[5], 13}, {kInf, 14},    {kPos[6], 14}, {kInf, 15}};
 static_assert((int)(kPos[0] * 4) == 1 && (int)(kPos[1] * 4) == 2 && (int)(kPos[2] * 4) == 3 &&
                   (int)(kPos[3] * 4) == 4 && (int)(kPos[4] * 4) == 5 &&
                   (int)(kPos[5] * 4) == 7 && (int)(kPos[6] * 4) == 9,
               "each threshold sits in the bin the table gives it");
 static_assert(kPos[0] * 4 != 1 && kPos[1] * 4 != 2 && kPos[2] * 4 != 3 && kPos[3] * 4 != 4 &&
                   kPos[4] * 4 != 5 && kPos[5] * 4 != 7 && kPos[6] * 4 != 9,
-              "no threshold on a bin boundary");
+              "no threshold but 0 on a bin boundary");
 
 // The codec's level of z = y * (1/scale): #{i : t_i < z} (NaN -> 0). lut:
-// kBins staged in LDS.
+// kBins staged in LDS. The bin is the truncated 4z + 11 (a negative sum and a
+// NaN give 0); where that sum's rounding crosses a bin's end, no threshold
+// lies between z and the end, so both bins give the same count.
 __device__ __forceinline__ uint32_t level_of(float z, const LevelBin* lut)
 {
-    const float a = fabsf(z);
-    // for z < 0 the count is 7 - #{t_k <= |z|} = 7 - #{t_k < nextup(|z|)}
-    const float up = __uint_as_float(min(__float_as_uint(a) + 1u, 0x7F800000u));
-    const bool neg = z < 0.0f;
-    const float b = neg ? up : a;
-    // truncation: a NaN gives bin 0, +inf saturates to the last bin
-    const uint32_t bin = min(__float2uint_rz(b * 4.0f), (uint32_t)(kLevelBins - 1));
-    const LevelBin e = lut[bin];
-    const uint32_t c = e.below + (e.inside < b ? 1u : 0u);
-    return z > 0.0f ? 8u + c : neg ? 7u - c : (z == 0.0f ? 7u : 0u);
+    // 8 bytes an entry: the byte offset is the truncated 32z + 88, its low
+    // bits dropped
+    const uint32_t u = min(__float2uint_rz(__builtin_fmaf(z, 32.0f, 88.0f)), 8u * kLevelBins - 1u);
+    const LevelBin e = *(const LevelBin*)((const char*)lut + (u & ~7u));
+    return e.below + (e.inside < z ? 1u : 0u);
 }
 
+// Sixteen (token, kv head) items per workgroup, both planes of an item on its
+// 16 lanes: the two rows share the index arithmetic, the slot, the signs and
+// the scale's square root and division. Bound by the vector ALU: the codec's
+// arithmetic is about 240 instructions a row against 330 bytes of traffic at
+// d = 128. 4096 BF16 tokens x 8 heads of 128: 11.7 us with one row a lane and
+// bins of |z| (17 instructions a level), 9.1 with two rows and signed bins
+// (6 and an LDS read), 8.4 with the shared scale and a multiplier for item / H;
+// 16384 tokens 32 -> 21.5 us (3.9 TB/s).
 template <int D, int IN_BF16>
 __global__ __launch_bounds__(kRmsThreads) void rms_writer(
     const uint16_t* __restrict__ key, const uint16_t* __restrict__ value,
     int8_t* __restrict__ key_cache, int8_t* __restrict__ value_cache,
     float* __restrict__ scale_cache, const int32_t* __restrict__ slots,
-    const float* __restrict__ pi_signs, uint32_t tokens, uint32_t H, uint64_t slot_count,
-    float inv_sqrt_len)
+    const float* __restrict__ pi_signs, uint32_t tokens, uint32_t H, uint32_t h_magic,
+    uint32_t h_shift, uint64_t slot_count, float inv_sqrt_len)
 {
     constexpr int CPL = D / kRowLanes;
     const int lane = threadIdx.x & (kRowLanes - 1);
     const int l = row_lane(lane);  // logical lane: channels l*CPL ..
     // the level search's bins, staged before any lane leaves
     __shared__ LevelBin lut[kLevelBins];
-    if (threadIdx.x == 0) {
-#pragma unroll
-        for (int b = 0; b < kLevelBins; ++b) lut[b] = kBins[b];
-    }
+    if (threadIdx.x < kLevelBins) lut[threadIdx.x] = kBins[threadIdx.x];
     __syncthreads();
-    const uint64_t row = (uint64_t)blockIdx.x * (kRmsThreads / kRowLanes) + threadIdx.x / kRowLanes;
-    const uint32_t planes = 2 * H;
-    const uint64_t rows = (uint64_t)tokens * planes;
-    if (row >= rows) return;
-    // 32-bit division when every row index fits (a uniform branch)
-    const uint32_t t = rows <= 0xffffffffull ? (uint32_t)row / planes : (uint32_t)(row / planes);
-    const uint32_t plane = (uint32_t)row - t * planes;
-    const uint32_t h = plane < H ? plane : plane - H;
+    const uint64_t item = (uint64_t)blockIdx.x * (kRmsThreads / kRowLanes) + threadIdx.x / kRowLanes;
+    const uint64_t items = (uint64_t)tokens * H;
+    if (item >= items) return;
+    // item / H by the launch's multiplier when every item is below 2^31 (a
+    // uniform branch)
+    const uint32_t t = items <= 0x7fffffffull
+                           ? (uint32_t)(((uint64_t)(uint32_t)item * h_magic) >> h_shift)
+                           : (uint32_t)(item / H);
+    const uint32_t h = (uint32_t)(item - (uint64_t)t * H);
     const int32_t slot = slots[t];
-    // the row's channels lane*CPL .. +CPL: one vector load, and the signs
-    const uint16_t* src = (plane < H ? key : value) + ((uint64_t)t * H + h) * D + l * CPL;
-    uint16_t raw[CPL];
-    if constexpr (CPL == 4) {
-        const uint2 w = *(const uint2*)src;
-        raw[0] = w.x & 0xffff; raw[1] = w.x >> 16; raw[2] = w.y & 0xffff; raw[3] = w.y >> 16;
-    } else {
+    // the rows' channels l*CPL .. +CPL, and the signs
+    uint32_t raw[2][CPL / 2];
+    __builtin_memcpy(raw[0], key + item * D + l * CPL, CPL * 2);
+    __builtin_memcpy(raw[1], value + item * D + l * CPL, CPL * 2);
+    float sg[CPL];
 #pragma unroll
-        for (int q = 0; q < CPL / 8; ++q) {
-            const uint4 w = *(const uint4*)(src + 8 * q);
-            const uint32_t u[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                raw[8 * q + 2 * k] = u[k] & 0xffff;
-                raw[8 * q + 2 * k + 1] = u[k] >> 16;
-            }
-        }
-    }
-    float sg[CPL], v[CPL];
-#pragma unroll
-    for (int j = 0; j < CPL; ++j) {
-        sg[j] = pi_signs[l * CPL + j];
-        v[j] = IN_BF16 ? bf16_to_f32(raw[j]) : (float)__builtin_bit_cast(_Float16, raw[j]);
-    }
+    for (int j = 0; j < CPL; ++j) sg[j] = pi_signs[l * CPL + j];
     if (slot < 0 || (uint64_t)slot >= slot_count) return;  // a pad token or a slot past the pool
 
     // ApplyPi: signs, FWHT at strides 1 .. D/2, x inv_sqrt_len, signs. The
-    // FWHT's cross-lane stages run on sign-tracked values (row_fmac_stage):
-    // v holds sigma * y afterwards, sigma = row_sigma(l)
+    // first signs flip the 16-bit values' sign bits, two at a time. The FWHT's
+    // cross-lane stages run on sign-tracked values (row_fmac_stage): v holds
+    // sigma * y afterwards, sigma = row_sigma(l)
+    float v[2][CPL];
 #pragma unroll
-    for (int j = 0; j < CPL; ++j) v[j] = v[j] * sg[j];
+    for (int j = 0; j < CPL; j += 2) {
+        const uint32_t flip = (__float_as_uint(sg[j]) & 0x80000000u) >> 16 |
+                              (__float_as_uint(sg[j + 1]) & 0x80000000u);
 #pragma unroll
-    for (int s = 1; s < D; s <<= 1) {
-        if (s < CPL) {
-#pragma unroll
-            for (int j = 0; j < CPL; ++j) {
-                if (j & s) continue;
-                const float a = v[j];
-                const float b = v[j + s];
-                v[j] = b + a;
-                v[j + s] = a - b;
+        for (int r = 0; r < 2; ++r) {
+            const uint32_t w = raw[r][j / 2] ^ flip;
+            if constexpr (IN_BF16) {
+                v[r][j] = __uint_as_float(w << 16);
+                v[r][j + 1] = __uint_as_float(w & 0xffff0000u);
+            } else {
+                v[r][j] = (float)__builtin_bit_cast(_Float16, (uint16_t)w);
+                v[r][j + 1] = (float)__builtin_bit_cast(_Float16, (uint16_t)(w >> 16));
             }
-        } else {
-            const int k = __builtin_ctz(s / CPL);
-            row_fmac_stage<CPL>(v, ((l >> k) & 1) ? -1.0f : 1.0f, k);
         }
     }
 #pragma unroll
-    for (int j = 0; j < CPL; ++j) v[j] = (v[j] * inv_sqrt_len) * sg[j];
-
-    // scale = sqrt(sum y^2) * inv_sqrt_len + eps: per-lane sequential sum,
-    // then the tree over logical lanes l ^ 1, l ^ 2, l ^ 4, l ^ 8 ((sigma y)^2
-    // is y^2 exactly)
-    float ss = v[0] * v[0];
+    for (int s = 1; s < D; s <<= 1) {
 #pragma unroll
-    for (int j = 1; j < CPL; ++j) ss = ss + v[j] * v[j];
+        for (int r = 0; r < 2; ++r) {
+            if (s < CPL) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) row_add1(ss, k);
-    const float scale = sqrt_rn(ss) * inv_sqrt_len + kRmsEps;
-    // sigma rides on the reciprocal: (sigma y) * (sigma r) rounds as y * r
-    const float rcp = row_sigma(l) * __fdiv_rn(1.0f, scale);
-
-    // levels, packed (even | odd << 4) ^ 0x80 -- the -128 bias of the int8 byte
-    uint32_t pk[CPL / 8 > 0 ? CPL / 8 : 1] = {};
-#pragma unroll
-    for (int j = 0; j < CPL; ++j) {
-        const uint32_t q = level_of(v[j] * rcp, lut);
-        pk[j / 8] |= q << (4 * (j % 8));
+                for (int j = 0; j < CPL; ++j) {
+                    if (j & s) continue;
+                    const float a = v[r][j];
+                    const float b = v[r][j + s];
+                    v[r][j] = b + a;
+                    v[r][j + s] = a - b;
+                }
+            } else {
+                const int k = __builtin_ctz(s / CPL);
+                row_fmac_stage<CPL>(v[r], ((l >> k) & 1) ? -1.0f : 1.0f, k);
+            }
+        }
     }
-    int8_t* dst = (plane < H ? key_cache : value_cache) + ((uint64_t)slot * H + h) * (D / 2) +
-                  l * (CPL / 2);
-    if constexpr (CPL == 4) {
-        *(uint16_t*)dst = (uint16_t)(pk[0] ^ 0x8080u);
-    } else if constexpr (CPL == 8) {
-        *(uint32_t*)dst = pk[0] ^ 0x80808080u;
-    } else {
-        *(uint2*)dst = make_uint2(pk[0] ^ 0x80808080u, pk[1] ^ 0x80808080u);
+    // x inv_sqrt_len, then the sign: one product with the signed factor (the
+    // sign is +-1, so the rounding is the same)
+#pragma unroll
+    for (int j = 0; j < CPL; ++j) sg[j] = inv_sqrt_len * sg[j];
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+#pragma unroll
+        for (int j = 0; j < CPL; ++j) v[r][j] = v[r][j] * sg[j];
     }
-    // the slot's scale record: this plane's scale, and its share of the zero padding
-    const uint32_t ssf = (planes + 7u) / 8u * 8u;
+
+    // scale = sqrt(sum y^2) * inv_sqrt_len + eps: per-lane sequential sum, then
+    // the tree over logical lanes l ^ 1, l ^ 2, l ^ 4, l ^ 8 ((sigma y)^2 is
+    // y^2 exactly). Even lanes then finish the key row, odd lanes the value row.
+    float ss[2];
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        ss[r] = v[r][0] * v[r][0];
+#pragma unroll
+        for (int j = 1; j < CPL; ++j) ss[r] = ss[r] + v[r][j] * v[r][j];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) row_add1(ss[r], k);
+    }
+    const float scale = sqrt_rn((lane & 1) ? ss[1] : ss[0]) * inv_sqrt_len + kRmsEps;
+    const uint32_t ssf = (2u * H + 7u) / 8u * 8u;
     float* rec = scale_cache + (uint64_t)slot * ssf;
-    if (lane == 0) {
-        rec[plane] = scale;
-    } else {
-        const uint32_t pad = planes + plane * (kRowLanes - 1) + (lane - 1);
-        if (pad < ssf) rec[pad] = 0.0f;
+    if (lane < 2) rec[lane * H + h] = scale;
+    // sigma rides on the reciprocal: (sigma y) * (sigma r) rounds as y * r
+    const int rcp = __float_as_int(__fdiv_rn(1.0f, scale));
+    const float sigma = row_sigma(l);
+    const float rcps[2] = {
+        sigma * __int_as_float(__builtin_amdgcn_mov_dpp(rcp, 0xA0, 0xf, 0xf, true)),   // lanes 0,0,2,2
+        sigma * __int_as_float(__builtin_amdgcn_mov_dpp(rcp, 0xF5, 0xf, 0xf, true))};  // lanes 1,1,3,3
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        // levels, packed (even | odd << 4) ^ 0x80 -- the -128 bias of the int8 byte
+        uint32_t pk[CPL / 8 > 0 ? CPL / 8 : 1] = {};
+#pragma unroll
+        for (int j = 0; j < CPL; ++j) pk[j / 8] |= level_of(v[r][j] * rcps[r], lut) << (4 * (j % 8));
+        int8_t* dst = (r == 0 ? key_cache : value_cache) + ((uint64_t)slot * H + h) * (D / 2) +
+                      l * (CPL / 2);
+        if constexpr (CPL == 4) {
+            *(uint16_t*)dst = (uint16_t)(pk[0] ^ 0x8080u);
+        } else if constexpr (CPL == 8) {
+            *(uint32_t*)dst = pk[0] ^ 0x80808080u;
+        } else {
+            *(uint2*)dst = make_uint2(pk[0] ^ 0x80808080u, pk[1] ^ 0x80808080u);
+        }
     }
+    // the slot's scale record ends in at most 7 zeros, head 0's to write
+    if (h == 0 && lane > 0 && 2u * H + lane - 1u < ssf) rec[2u * H + lane - 1u] = 0.0f;
 }
 
 // Dequantize4Bit: four packed bytes -> eight centroids per lane, grid-stride.
@@ -261,14 +277,19 @@ hipError_t launch_rms_writer_t(hipStream_t stream, int in_bf16, const uint16_t* 
                                const int32_t* slots, const float* signs, uint32_t tokens,
                                uint32_t H, uint64_t slot_count, float isl)
 {
-    const uint64_t rows = (uint64_t)tokens * 2 * H;
-    const uint32_t blocks = (uint32_t)((rows + kRmsThreads / kRowLanes - 1) / (kRmsThreads / kRowLanes));
+    const uint64_t items = (uint64_t)tokens * H;
+    const uint32_t blocks = (uint32_t)((items + kRmsThreads / kRowLanes - 1) / (kRmsThreads / kRowLanes));
+    // n / H for n < 2^31: (n * magic) >> shift, magic = floor(2^shift / H) + 1
+    // with 2^(shift - 31) the power of two at or above H
+    uint32_t shift = 31;
+    while (shift < 63 && (1ull << (shift - 31)) < H) ++shift;
+    const uint32_t magic = H == 1 ? 0x80000000u : (uint32_t)((1ull << shift) / H + 1);
     if (in_bf16)
         hipLaunchKernelGGL((rms_writer<D, 1>), dim3(blocks), dim3(kRmsThreads), 0, stream, key,
-                           value, kc, vc, sc, slots, signs, tokens, H, slot_count, isl);
+                           value, kc, vc, sc, slots, signs, tokens, H, magic, shift, slot_count, isl);
     else
         hipLaunchKernelGGL((rms_writer<D, 0>), dim3(blocks), dim3(kRmsThreads), 0, stream, key,
-                           value, kc, vc, sc, slots, signs, tokens, H, slot_count, isl);
+                           value, kc, vc, sc, slots, signs, tokens, H, magic, shift, slot_count, isl);
     return hipGetLastError();
 }
 

@@ -156,3 +156,11 @@ def hadamard(n):
     while h.shape[0] < n:
         h = np.block([[h, h], [h, -h]])
     return h
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("T,H", [(2, 1), (17, 1), (33, 5), (5, 16), (7, 31), (1, 4)])
+def test_writer_item_and_scale_record_edges(tq4, oracle, T, H, d):
+    """Item counts around a workgroup's sixteen, head counts that the index
+    multiplier and the scale record's zero padding treat differently."""
+    run_case(tq4, oracle, max(T, 2), H, d, 16, 4, bool(T % 2), seed=T * 100 + H + d)
