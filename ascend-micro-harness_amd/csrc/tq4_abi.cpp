@@ -34,6 +34,10 @@ size_t ticket_bytes(uint32_t num_seqs, uint32_t num_kv_heads)
            ~(size_t)255;
 }
 
+// The tail's counters are placed from the workspace's end: a size that is no
+// multiple of four would put the atomics across word boundaries.
+size_t whole_words(size_t bytes) { return bytes & ~(size_t)3; }
+
 int writer_checks(const void* key, const void* value, const int8_t* key_cache,
                   const int8_t* value_cache, const float* scale_cache, const int32_t* slots,
                   const float* pi_signs, const int32_t* tables, uint32_t num_tokens,
@@ -239,6 +243,7 @@ int tq4_decode_poll_timeouts(void* stream, const void* workspace, size_t workspa
                              uint32_t num_seqs, uint32_t num_kv_heads, uint32_t* count)
 {
     if (!workspace || !count) return TQ4_ERR_NULL_POINTER;
+    workspace_bytes = whole_words(workspace_bytes);
     const size_t tail = ticket_bytes(num_seqs, num_kv_heads) + kQueueBytes;
     if (num_seqs == 0 || num_kv_heads == 0 || workspace_bytes < tail ||
         ((uintptr_t)workspace & 15u))
@@ -346,6 +351,7 @@ int tq4_paged_decode(void* stream, const uint16_t* q, const int8_t* key_cache,
     if (num_splits > 1) {
         const size_t need =
             tq4_decode_workspace_bytes(num_seqs, num_heads, num_kv_heads, head_size, num_splits);
+        workspace_bytes = whole_words(workspace_bytes);
         if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 15u))
             return TQ4_ERR_WORKSPACE;
         p.records = (float*)workspace;

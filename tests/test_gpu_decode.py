@@ -595,3 +595,21 @@ def test_record_chunk_edges(tq4, oracle, d, K, B):
     assert np.array_equal(outs[0], outs[2])
     assert tq4.decode_poll_timeouts(ws, B, H) == 0
     assert not torch.any(ws)
+
+
+def test_workspace_size_no_multiple_of_four(tq4, oracle):
+    """The counters sit at the workspace's end: a size with odd bytes at its
+    end is taken as whole words, so their atomics stay aligned."""
+    import torch
+    rng = np.random.default_rng(0x0DD)
+    Hq, H, d, S, K = 8, 2, 128, 16, 4
+    kc, vc, sc, tables, signs, isl = build_cache(oracle, rng, [300], H, d, S, 24)
+    q = f32_to_bf16(rng.standard_normal((1, Hq, d)).astype(np.float32))
+    args = [dev(q), dev(kc), dev(vc), dev(sc), dev(tables), dev(np.array([300], np.int32)),
+            dev(signs)]
+    whole = tq4.decode_workspace(1, Hq, H, d, K)
+    odd = torch.zeros(whole.numel() + 7, dtype=torch.uint8, device="cuda")
+    outs = [host(tq4.paged_decode(*args, H, S, 24, workspace=w, num_splits=K,
+                                  inv_sqrt_len=float(isl))) for w in (whole, odd, odd)]
+    assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], outs[2])
+    assert tq4.decode_poll_timeouts(odd, 1, H) == 0
