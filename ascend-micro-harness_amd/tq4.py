@@ -47,6 +47,11 @@ _I32 = C.c_int
 _SZ = C.c_size_t
 
 _lib = None
+# The native argument checks and launches (csrc/tq4_host.cpp), once the library
+# is loaded. Each function takes a call whole when it is plainly valid and
+# returns None, without any effect, when it is not: the Python below then makes
+# the call or refuses it.
+_fast = None
 
 
 class TQ4Error(ValueError):
@@ -119,7 +124,30 @@ def lib():
     L.tq4_fp8_e4m3_round.restype = _I32
     L.tq4_fp8_e4m3_round.argtypes = [_P, _P, _P, C.c_uint64]
     _lib = L
+    _bind_host(L)
     return L
+
+
+def _bind_host(L):
+    global _fast
+    if not os.path.exists(os.path.join(_HERE, "_tq4_host.so")):
+        return
+    from . import _tq4_host as host
+    host.bind({n: C.cast(getattr(L, n), _P).value for n in (
+        "tq4_reshape_and_cache_a8", "tq4_reshape_and_cache_bf16", "tq4_reshape_scatter",
+        "tq4_decode_auto_splits", "tq4_paged_decode", "tq4_paged_decode_partials",
+        "tq4_splitk_combine", "tq4_rms_reshape_and_cache", "tq4_icdf_quantize",
+        "tq4_lloydmax_quantize", "tq4_kv4fp8_workspace_bytes", "tq4_kv4fp8_decode",
+        "tq4_kv4fp8_decode_raw_query")})
+    _fast = host
+
+
+def _done(r, what):
+    """Whether the native call took the call (r is not None); a refused launch
+    raises."""
+    if type(r) is int and r != 0:
+        _check(r, what)
+    return r is not None
 
 
 def status_string(status):
@@ -186,6 +214,11 @@ def reshape_and_cache_a8(key, value, key_cache, value_cache, scale_cache, slot_m
                          tokens_per_core=16, inv_sqrt_len=None, reuse_mode4_flags=True,
                          stream=None):
     """INT8 K/V [num_tokens][num_kv_heads][head_size] -> TQ4 cache, whole strips."""
+    if _fast is not None and _done(_fast.reshape_and_cache(
+            True, key, value, key_cache, value_cache, scale_cache, slot_mapping, pi_signs, tables,
+            block_size, num_blocks, tokens_per_core, inv_sqrt_len, reuse_mode4_flags, stream),
+            "reshape_and_cache_a8"):
+        return None
     return _reshape_and_cache(lib().tq4_reshape_and_cache_a8, "reshape_and_cache_a8", torch.int8,
                               key, value, key_cache, value_cache, scale_cache, slot_mapping,
                               pi_signs, tables, num_blocks, block_size, tokens_per_core,
@@ -197,6 +230,11 @@ def reshape_and_cache_bf16(key, value, key_cache, value_cache, scale_cache, slot
                            tokens_per_core=16, inv_sqrt_len=None, reuse_mode4_flags=True,
                            stream=None):
     """BF16 K/V [num_tokens][num_kv_heads][head_size] -> TQ4 cache, whole strips."""
+    if _fast is not None and _done(_fast.reshape_and_cache(
+            False, key, value, key_cache, value_cache, scale_cache, slot_mapping, pi_signs, tables,
+            block_size, num_blocks, tokens_per_core, inv_sqrt_len, reuse_mode4_flags, stream),
+            "reshape_and_cache_bf16"):
+        return None
     return _reshape_and_cache(lib().tq4_reshape_and_cache_bf16, "reshape_and_cache_bf16",
                               torch.bfloat16, key, value, key_cache, value_cache, scale_cache,
                               slot_mapping, pi_signs, tables, num_blocks, block_size,
@@ -240,6 +278,11 @@ def reshape_scatter(key, value, key_cache, value_cache, scale_cache, slot_mappin
                     inv_sqrt_len=None, stream=None):
     """BF16 tokens at arbitrary slots; items are (request, kv_head)."""
     what = "reshape_scatter"
+    if _fast is not None and _done(_fast.reshape_scatter(
+            key, value, key_cache, value_cache, scale_cache, slot_mapping, pi_signs, cu_seqlens,
+            launch_probe, num_requests, block_size, num_blocks, item_begin, item_count, block_dim,
+            inv_sqrt_len, stream), what):
+        return
     _need(what, "key", key, (torch.bfloat16,), ndim=3)
     _need(what, "value", value, (torch.bfloat16,), numel=key.numel())
     num_tokens, num_kv_heads, head_size = key.shape
@@ -360,6 +403,12 @@ def paged_decode(q, key_cache, value_cache, scale_cache, block_tables, context_l
                  num_splits=0, scale=None, inv_sqrt_len=None, output_stage=1, flags=0,
                  stream=None):
     """Fused split-K decode: q [B][Hq][d] bf16 -> out [B][Hq][d] bf16."""
+    if _fast is not None:
+        r = _fast.paged_decode(q, key_cache, value_cache, scale_cache, block_tables, context_lens,
+                               pi_signs, num_kv_heads, block_size, num_blocks, out, workspace,
+                               gate, num_splits, scale, inv_sqrt_len, output_stage, flags, stream)
+        if _done(r, "paged_decode"):
+            return r
     _check_decode_inputs("paged_decode", q, key_cache, value_cache, scale_cache, block_tables,
                          context_lens, pi_signs, num_kv_heads, block_size, num_blocks,
                          pi_needed=output_stage >= 1 or not (flags & TQ4_DECODE_QUERY_ROTATED))
@@ -441,6 +490,13 @@ def paged_decode_partials(q, key_cache, value_cache, scale_cache, block_tables, 
                           pi_signs, num_kv_heads, block_size, num_blocks, num_splits,
                           workspace=None, scale=None, inv_sqrt_len=None, flags=0, stream=None):
     """Partial records [B][Hq][K][d+4] = (m, l, 0, 0, acc[d]) per split."""
+    if _fast is not None:
+        r = _fast.paged_decode_partials(
+            q, key_cache, value_cache, scale_cache, block_tables, context_lens, pi_signs,
+            num_kv_heads, block_size, num_blocks, num_splits, workspace, scale, inv_sqrt_len,
+            flags, stream)
+        if _done(r, "paged_decode_partials"):
+            return r
     _check_decode_inputs("paged_decode_partials", q, key_cache, value_cache, scale_cache,
                          block_tables, context_lens, pi_signs, num_kv_heads, block_size,
                          num_blocks, pi_needed=not (flags & TQ4_DECODE_QUERY_ROTATED))
@@ -472,6 +528,11 @@ def splitk_combine(workspace, pi_signs, num_seqs, num_heads, head_size, num_spli
                    gate=None, inv_sqrt_len=None, output_stage=1, stream=None):
     """LSE combine + egress of partial records into BF16 [B][Hq][d]."""
     what = "splitk_combine"
+    if _fast is not None:
+        r = _fast.splitk_combine(workspace, pi_signs, num_seqs, num_heads, head_size, num_splits,
+                                 out, gate, inv_sqrt_len, output_stage, stream)
+        if _done(r, what):
+            return r
     rows = num_seqs * num_heads
     _need(what, "workspace", workspace, (torch.float32,),
           min_numel=rows * num_splits * (head_size + 4))
@@ -507,6 +568,10 @@ def rms_reshape_and_cache(key, value, key_cache, value_cache, scale_cache, slot_
     FP16/BF16 K/V [tokens][kv_heads][head_size] -> int8 rows [slot][kv_heads]
     [head_size/2] and the scale record [slot][ceil(2 kv_heads / 8) * 8]."""
     what = "rms_reshape_and_cache"
+    if _fast is not None and tables is None and _done(_fast.rms_reshape_and_cache(
+            key, value, key_cache, value_cache, scale_cache, slot_mapping, pi_signs, block_size,
+            num_blocks, inv_sqrt_len, block_dim, tokens_per_core, stream), what):
+        return
     _need(what, "key", key, (torch.float16, torch.bfloat16), ndim=3)
     _need(what, "value", value, (key.dtype,), numel=key.numel())
     T, H, d = key.shape
@@ -551,6 +616,10 @@ def rms_dequantize(packed, out=None, stream=None):
 def icdf_quantize(x, out=None, stream=None):
     """FP16 or BF16 values (a multiple of 1024) -> packed signed INT4 codes of
     RNE(14 sigmoid(x) - 7), element 2j in the low nibble of byte j."""
+    if _fast is not None:
+        r = _fast.icdf_quantize(x, out, stream)
+        if _done(r, "icdf_quantize"):
+            return r
     _dev(x, "x")
     if x.dtype not in (torch.float16, torch.bfloat16):
         raise ValueError("icdf_quantize: x must be float16 or bfloat16")
@@ -568,6 +637,10 @@ def lloydmax_quantize(src, bits=4, mode=0, dst=None, codes=None, stream=None):
     """The Lloyd-Max leaf and its companions (mode as tq4_lloydmax_quantize):
     0/1 Lloyd-Max, 2 Gaussian-CDF compander, 3 ICDF (FP16 src), 4/5 decode of
     packed codes. Returns (dst, codes)."""
+    if _fast is not None:
+        r = _fast.lloydmax_quantize(src, bits, mode, dst, codes, stream)
+        if _done(r, "lloydmax_quantize"):
+            return r
     _dev(src, "src")
     if mode >= 4:
         n = src.numel() * 8 // bits
@@ -714,6 +787,13 @@ def kv4fp8_decode(query, key_cache, value_cache, scales, block_table, context_le
     """The pre-rotated entry: query FP32 [T][Hq][256] -> out [T][Hq][256] (FP16/BF16).
     test_flags: the bounded wait's test hooks (TQ4_KV4FP8_TEST_*), 0 in use."""
     what = "kv4fp8_decode"
+    if _fast is not None and not test_flags:
+        r = _fast.kv4fp8_decode(False, query, None, key_cache, value_cache, scales, block_table,
+                                context_lens, kv_heads, block_size, num_blocks, None, 0, None, out,
+                                out_dtype is torch.bfloat16, workspace, splits, heads_per_task,
+                                fused_context_limit, scale, inv_sqrt_len, stream)
+        if _done(r, what):
+            return r
     _need(what, "query", query, (torch.float32,), ndim=3)
     _kv4_check(what, query, key_cache, value_cache, scales, block_table, context_lens,
                kv_heads, block_size, num_blocks)
@@ -747,6 +827,13 @@ def kv4fp8_decode_raw_query(raw_query, pi_signs, key_cache, value_cache, scales,
     """The raw-query entry: raw_query FP16/BF16 [T][Hq][256] in the original
     basis -> out (same element type); query_out receives the rotated FP32 query."""
     what = "kv4fp8_decode_raw_query"
+    if _fast is not None:
+        r = _fast.kv4fp8_decode(True, raw_query, pi_signs, key_cache, value_cache, scales,
+                                block_table, context_lens, kv_heads, block_size, num_blocks, gate,
+                                output_stage, query_out, out, False, workspace, splits,
+                                heads_per_task, fused_context_limit, scale, inv_sqrt_len, stream)
+        if _done(r, what):
+            return r
     _need(what, "raw_query", raw_query, (torch.float16, torch.bfloat16), ndim=3)
     _kv4_check(what, raw_query, key_cache, value_cache, scales, block_table, context_lens,
                kv_heads, block_size, num_blocks)
