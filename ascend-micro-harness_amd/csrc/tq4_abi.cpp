@@ -160,14 +160,19 @@ size_t tq4_decode_workspace_bytes(uint32_t num_seqs, uint32_t num_heads, uint32_
            kQueueBytes + ticket_bytes(num_seqs, num_kv_heads);
 }
 
-uint32_t tq4_decode_auto_splits(uint32_t num_seqs, uint32_t num_kv_heads,
-                                uint32_t max_blocks_per_seq, uint32_t block_size)
+namespace {
+
+// The split rule. filled: no second split wave for launches whose workgroups
+// already fill the last round of 256 CUs to 7/8 (for callers that know the
+// batch not to be skewed).
+uint32_t split_rule(uint32_t num_seqs, uint32_t num_kv_heads, uint32_t max_blocks_per_seq,
+                    uint32_t block_size, bool filled)
 {
     // Workgroups for half the CUs (256); for one per CU while each split
     // still holds 16 strips (20 when that takes the fused combine past one
-    // 16-split record chunk); for all their two slots when the splits would
-    // still be long (> 64 strips); splits of at most ~512 strips; never
-    // fewer than 16 strips per split, and at most 32 splits.
+    // 16-split record chunk, 8 for up to 8 splits); for all their two slots
+    // when the splits would still be long (> 64 strips); splits of at most
+    // ~512 strips; at most 32 splits.
     // - Each extra item costs a table and a first-strip round trip, a merge
     //   and a record, and the persistent kernel orders the last splits
     //   longest first, so a batch that already fills the slots runs best
@@ -177,6 +182,10 @@ uint32_t tq4_decode_auto_splits(uint32_t num_seqs, uint32_t num_kv_heads,
     //   from 12288 (16384: 10.7 against 11.6 us). Two sequences at ctx 4096
     //   and 8192, four at ctx 4096: one workgroup per CU, 11-16 % faster
     //   than half the CUs.
+    // - Contexts of 32 strips on take splits of 8 strips, up to 8 of them (one to eight
+    //   sequences x 8 KV heads, us with 16 / 8 strips a split: ctx 512 7.3 /
+    //   6.9, at d = 256 11.0 / 9.5; ctx 1024 7.4 / 7.0); 16 splits of 8
+    //   strips at ctx 2048 lose to 8 of 16 (7.5 / 7.3).
     // - More than 32 splits combine in two record chunks and measured 5-7 us
     //   slower than 32 at d = 128.
     const uint64_t strips = (uint64_t)max_blocks_per_seq * (block_size / kStrip);
@@ -185,8 +194,10 @@ uint32_t tq4_decode_auto_splits(uint32_t num_seqs, uint32_t num_kv_heads,
                                : 1;
     uint64_t k = (128 + items - 1) / items;
     const uint64_t per_cu = 256 / items;
-    if (per_cu > k && strips >= (per_cu > 16 ? 20 : 16) * per_cu) k = per_cu;
-    if (strips > 64 * k) {
+    const uint64_t least = per_cu > 16 ? 20 : per_cu > 8 || per_cu < 4 ? 16 : 8;
+    if (per_cu > k && strips >= least * per_cu) k = per_cu;
+    const uint64_t rounds = (items * k + 255) / 256;
+    if (strips > 64 * k && !(filled && items * k * 8 >= rounds * 256 * 7)) {
         uint64_t more = (512 + items - 1) / items;
         const uint64_t by_work = (strips + 63) / 64;
         if (more > by_work) more = by_work;
@@ -194,7 +205,9 @@ uint32_t tq4_decode_auto_splits(uint32_t num_seqs, uint32_t num_kv_heads,
     }
     const uint64_t k_len = (strips + 511) / 512;
     if (k < k_len) k = k_len;
-    const uint64_t by_len = strips / 16 > 0 ? strips / 16 : 1;
+    uint64_t by_len = strips / 16;
+    if (strips >= 32 && by_len < 8) by_len = strips / 8 < 8 ? strips / 8 : 8;
+    if (by_len < 1) by_len = 1;
     if (k > by_len) k = by_len;
     if (k > 32) k = 32;
     // one split stages at most TQ4_MAX_SPLIT_STRIPS strips of its window
@@ -205,19 +218,20 @@ uint32_t tq4_decode_auto_splits(uint32_t num_seqs, uint32_t num_kv_heads,
     return (uint32_t)k;
 }
 
+}  // namespace
+
+uint32_t tq4_decode_auto_splits(uint32_t num_seqs, uint32_t num_kv_heads,
+                                uint32_t max_blocks_per_seq, uint32_t block_size)
+{
+    return split_rule(num_seqs, num_kv_heads, max_blocks_per_seq, block_size, false);
+}
+
 uint32_t tq4_decode_auto_splits_lens(uint32_t num_seqs, uint32_t num_kv_heads,
                                      uint32_t max_blocks_per_seq, uint32_t block_size,
                                      const int32_t* context_lens)
 {
-    uint32_t k = tq4_decode_auto_splits(num_seqs, num_kv_heads, max_blocks_per_seq, block_size);
-    if (!context_lens || num_seqs == 0 || num_kv_heads == 0) return k;
-    // A ragged batch (longest context >= 1.6 x the mean) whose (seq, kv head)
-    // items fill the resident slots (512 at d <= 128) between half and one
-    // and a half times: one item per (seq, kv head) leaves the launch waiting
-    // on the longest sequences, so split them at least three ways. Measured
-    // (64 x U[512, 8192]: 75.4 -> 72.3 us; 64 x U[128, 16384]: 133.3 ->
-    // 125.2; 80 x U[512, 8192]: 96.5 -> 92.7), while a uniform or mildly
-    // ragged batch (64 x 8192, 64 x U[2048, 8192]) runs best as it was.
+    if (!context_lens || num_seqs == 0 || num_kv_heads == 0)
+        return split_rule(num_seqs, num_kv_heads, max_blocks_per_seq, block_size, false);
     const uint64_t cap = (uint64_t)max_blocks_per_seq * block_size;
     uint64_t sum = 0, mx = 0;
     for (uint32_t b = 0; b < num_seqs; ++b) {
@@ -226,10 +240,30 @@ uint32_t tq4_decode_auto_splits_lens(uint32_t num_seqs, uint32_t num_kv_heads,
         sum += c;
         if (c > mx) mx = c;
     }
+    // Unless one sequence is several times the mean, workgroups that fill the
+    // CUs are not split again: a second wave of shorter items costs more than
+    // it evens out. Us with / without the second split, lengths spread over
+    // half to the whole of the longest: 4 sequences x 8 KV heads at ctx 12000
+    // 16.1 / 13.0 (d = 256 35.3 / 22.3), 8 at 12000 20.9 / 18.1 (46.8 / 36.4),
+    // 16 at 4096 15.3 / 14.6 (36.3 / 28.7), 32 at 2048 17.4 / 15.5 (44.8 /
+    // 31.8); 12 sequences (fill 3/4) still want it: 26.6 against 29.1.
+    uint32_t k = split_rule(num_seqs, num_kv_heads, max_blocks_per_seq, block_size,
+                            mx * num_seqs < 3 * sum);
+    // A ragged batch (longest context >= 1.6 x the mean) whose (seq, kv head)
+    // items fill the resident slots (512 at d <= 128) between half and one
+    // and a half times: one item per (seq, kv head) leaves the launch waiting
+    // on the longest sequences, so split them at least three ways, four when
+    // a longest item alone fills its CU. Measured (64 x U[512, 8192]: 75.4 ->
+    // 72.3 us; 64 x U[128, 16384]: 133.3 -> 125.2; 80 x U[512, 8192]: 96.5 ->
+    // 92.7; 32 x U[1200, 12000]: 58.1 -> 52.9), while a uniform or mildly
+    // ragged batch (64 x 8192, 64 x U[2048, 8192]) and short contexts (40 x
+    // U[100, 1024]: 12.9 against 17.3) run best as they are.
     const uint64_t items = (uint64_t)num_seqs * num_kv_heads;
-    if (sum > 0 && items * 2 > 512 && items * 2 <= 3 * 512 && mx * num_seqs * 5 >= sum * 8 &&
-        k < 3 && max_blocks_per_seq >= 3)
-        k = 3;
+    const bool ragged = sum > 0 && mx * num_seqs * 5 >= sum * 8;
+    const uint32_t want = items > 256 && items <= 768 && mx >= 192 * kStrip    ? 3
+                          : items > 192 && items <= 256 && mx >= 512 * kStrip ? 4
+                                                                              : 1;
+    if (ragged && k < want && max_blocks_per_seq >= want) k = want;
     return k;
 }
 

@@ -184,10 +184,12 @@ uint32_t tq4_decode_auto_splits(uint32_t num_seqs, uint32_t num_kv_heads,
  * workspace that tq4_paged_decode_partials has written since must be zeroed
  * again before tq4_paged_decode uses it. */
 /* tq4_decode_auto_splits for a caller that holds the context lengths on the
- * host (context_lens: num_seqs host integers; NULL gives the plain rule): a
- * ragged batch (longest >= 1.6 x mean) whose num_seqs * num_kv_heads lies
- * between 256 and 768 takes at least 3 splits. No reference counterpart (the
- * reference's callers pass their split count). */
+ * host (context_lens: num_seqs host integers; NULL gives the plain rule).
+ * Unless the longest is 3 times the mean, a batch whose workgroups fill the
+ * CUs is not split further; a ragged batch (longest >= 1.6 x mean) of 257 to
+ * 768 (seq, kv head) items takes at least 3 splits when its longest context
+ * has 192 strips, one of 193 to 256 items at least 4 from 512 strips on. No
+ * reference counterpart (the reference's callers pass their split count). */
 uint32_t tq4_decode_auto_splits_lens(uint32_t num_seqs, uint32_t num_kv_heads,
                                      uint32_t max_blocks_per_seq, uint32_t block_size,
                                      const int32_t* context_lens);

@@ -305,3 +305,33 @@ def test_floor_library_refuses_other_geometry():
         setattr(e, field, bad)
         assert fl.tq4_floor_scatter_launch(None, C.addressof(e)) == -1, field
     assert fl.tq4_floor_scatter_launch(None, None) == -1
+
+
+def test_auto_splits_short_filled_and_ragged(lib):
+    """The split rules' edges: 32-strip contexts, batches whose workgroups fill
+    the CUs (with and without a skewed length), ragged batches long and short."""
+    import numpy as np
+    f, g = lib.tq4_decode_auto_splits, lib.tq4_decode_auto_splits_lens
+    f.restype = g.restype = C.c_uint32
+    g.argtypes = [C.c_uint32] * 4 + [C.c_void_p]
+
+    def lens(b, mb, ls):
+        a = np.array(ls, np.int32)
+        return g(b, 8, mb, 16, a.ctypes.data)
+
+    assert [f(1, 8, p, 16) for p in (1, 16, 31, 32, 64, 128, 256)] == [1, 1, 1, 4, 8, 8, 16]
+    assert [f(1, 8, p, 128) for p in (1, 4, 8, 16)] == [1, 4, 8, 8]
+    # 8 sequences x 8 heads: 4 splits fill the CUs; the blind rule and a
+    # skewed batch keep 8
+    assert lens(8, 750, [12000] * 8) == 4
+    assert lens(8, 750, [12000] + [100] * 7) == 8 == f(8, 8, 750, 16)
+    # 12 sequences leave a quarter of the CUs idle: split on
+    assert lens(12, 750, [12000] * 12) == f(12, 8, 750, 16) == 6
+    # ragged: at least three (four) splits when the longest is long
+    ragged = [1200 + i * 10800 // 31 for i in range(32)]
+    assert lens(32, 750, ragged) == 4
+    assert lens(32, 500, [c // 8 for c in ragged]) == 1 and f(32, 8, 500, 16) == 2
+    assert lens(64, 256, [64 * (i + 1) for i in range(64)]) == 3
+    assert lens(64, 64, [16 * (i + 1) for i in range(64)]) == 1
+    for mb, page in ((8192, 16), (70000, 16), (3, 1024)):  # the staged window's bound
+        assert -(-mb // f(1, 1, mb, page)) * (page // 16) <= 2048
