@@ -796,7 +796,8 @@ __device__ __forceinline__ void park_rows(const RowState<D>& st, bool row_live, 
 // The end of one work item: merge the four waves' rows, then MODE 0 exports
 // the partial record; MODE 1 takes the split's place in the fused combine
 // (export, or finalise from LDS when it is the only live split, or combine as
-// the last ticket). region: the item's q staging / merge region.
+// the last ticket); MODE 2 exports a live split's record for the combine
+// launch behind it, or finalises the only live split. region: the item's q staging / merge region.
 template <int D, int MODE, bool OWN, int NS>
 __device__ __forceinline__ void finish_item(const DecodeParams& p, uint32_t seq, uint32_t kvh,
                                             uint32_t split, uint32_t k_live, uint32_t ticket,
@@ -898,12 +899,12 @@ __device__ __forceinline__ void finish_item(const DecodeParams& p, uint32_t seq,
         // window) finalises from LDS; otherwise every split exports and the
         // last ticket combines.
         const bool local = p.K == 1 || k_live == 1;
-        const int fl = *flag;
+        const int fl = MODE == 1 ? *flag : 0;
         const bool combiner = local || (fl & 1);
         float es[CC];
         if (!local && (fl & 2)) return;  // test hook: this record is never written
         if (!local && (!combiner || !OWN)) {
-            // ---- export this split's encoded record.
+            // ---- export this split's record (MODE 1: encoded).
             const __amdgpu_buffer_rsrc_t rsrc = records_rsrc(
                 p.records + (((size_t)seq * p.Hq + (size_t)kvh * G) * p.K + split) * RS);
             const uint32_t row_bytes = p.K * RS * 4u;
@@ -913,19 +914,19 @@ __device__ __forceinline__ void finish_item(const DecodeParams& p, uint32_t seq,
                 row_weights(r, f, M, L);
                 const float4 v = combined4(e4, f);
                 const float vv[4] = {v.x, v.y, v.z, v.w};
-                rec_store<4, true>(rsrc, r * row_bytes + (4 + ch) * 4u, vv);
+                rec_store<4, MODE == 1>(rsrc, r * row_bytes + (4 + ch) * 4u, vv);
                 if (ch == 0) {
                     // (m, l) only: the combiner clears what it reads, and a
                     // padding word left behind would read as a written word
                     // under another split count's record layout
                     const float h[2] = {M == -INFINITY ? kMasked : M * kLn2, L};
-                    rec_store<2, true>(rsrc, r * row_bytes, h);
+                    rec_store<2, MODE == 1>(rsrc, r * row_bytes, h);
                 }
             }
             TQ4_STAMP(6, TQ4_NOW);
             if (!combiner) return;
         }
-        if (!local) {
+        if (MODE == 1 && !local) {
             // ---- the combiner: poll the records of its rows and combine
             // them. With OWN its own record is never stored: its words are
             // made from LDS (the export's arithmetic, in the combine layout)
@@ -1000,7 +1001,8 @@ __device__ __forceinline__ void finish_item(const DecodeParams& p, uint32_t seq,
 }
 
 // One (seq, kv head, split) work item: MODE 0 exports the partial record,
-// MODE 1 is the fused path (ticket, export or local finish, combine).
+// MODE 1 is the fused path (ticket, export or local finish, combine), MODE 2
+// the first of two launches (export or local finish; combine_live_kernel).
 // OWN (MODE 1): the combining split keeps its own record in registers instead
 // of storing and polling it (the one-launch kernel; the persistent kernel
 // stores it, which keeps that kernel's register budget).
@@ -1078,7 +1080,7 @@ __device__ __forceinline__ void decode_item(const DecodeParams& p, const uint32_
     // split >= that count exactly when the window starts at or past ctx
     // (the window starts at page split * width), a test without divisions.
     uint32_t k_live = p.K;
-    if constexpr (MODE == 1) {
+    if constexpr (MODE != 0) {
         if (p.K > 1) {
             // 32-bit: its division runs while the table window is in flight
             const uint32_t width = p.max_blocks / p.K + (p.max_blocks % p.K != 0u);
@@ -1521,6 +1523,110 @@ __global__ __launch_bounds__(kThreads) void combine_kernel(DecodeParams p)
     egress_row<D>(v, es, gt, p.out + row * D, p.inv_sqrt_len, p.output_stage, lane);
 }
 
+// The second of the fused decode's two launches: one (seq, q head) row per
+// wave over the records of the sequence's live splits (the layout, the order
+// and the arithmetic of combine_records), zeroed once read. The first chunk's
+// loads do not wait for the context length that says which splits are live:
+// the records of dead ones are in range and all zero, and are selected out.
+// Rows of one live split (or none) are finished by the first launch.
+template <int D, int NS>
+__global__ __launch_bounds__(kThreads) void combine_live_kernel(DecodeParams p)
+{
+    constexpr int CC = D / 32;
+    constexpr int LD = CC >= 4 ? 4 : CC;  // floats per load
+    constexpr uint32_t kRowBytes = (D + 4) * 4;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t seq = blockIdx.x, head = blockIdx.y * kWaves + wave;  // no index division
+    if (head >= p.Hq) return;
+    const size_t row = (size_t)seq * p.Hq + head;
+    const int32_t ctx_raw = p.context_lens[seq];
+    const int c = lane & 31, ks = lane >> 5;
+    const __amdgpu_buffer_rsrc_t rsrc = records_rsrc(p.records + row * p.K * (D + 4));
+    uint32_t hw[NS][2], aw[NS][CC];
+    auto load_chunk = [&](uint32_t k0) {
+#pragma unroll
+        for (int i = 0; i < NS; ++i) {
+            const uint32_t o = min(k0 + ks + 2 * i, p.K - 1) * kRowBytes;
+            rec_load<2, false>(rsrc, o, hw[i]);
+#pragma unroll
+            for (int j = 0; j < CC; j += LD)
+                rec_load<LD, false>(rsrc, o + 4u * (4 + c * CC + j), &aw[i][j]);
+        }
+    };
+    load_chunk(0);
+    float es[CC], gt[CC], v[CC];
+    if (p.output_stage >= 1) load_lane_floats<D>(p.pi_signs, lane, es);
+    if (p.output_stage == 2) load_lane_floats<D>(p.gate + row * D, lane, gt);
+    // the live splits, as decode_item counts them
+    const uint32_t width = p.max_blocks / p.K + (p.max_blocks % p.K != 0u);
+    const uint64_t capacity = (uint64_t)p.max_blocks * p.S;
+    uint32_t ctx = ctx_raw < 0 ? 0u : (uint32_t)ctx_raw;
+    if (ctx > capacity) ctx = (uint32_t)capacity;
+    const uint32_t ctx_pages = ctx / p.S + (ctx % p.S != 0u);
+    const uint32_t k_live = ctx_pages / width + (ctx_pages % width != 0u);
+    if (k_live <= 1) return;
+    float M = -INFINITY, L = 0.0f, a[CC];
+#pragma unroll
+    for (int j = 0; j < CC; ++j) a[j] = 0.0f;
+    // The last chunk's records are zeroed under its arithmetic, earlier ones'
+    // after the loop: the next chunk's loads would wait for the stores. (A dead
+    // split's record is zero already.)
+    auto zero_chunk = [&](uint32_t k0) {
+#pragma unroll
+        for (int i = 0; i < NS; ++i) {
+            const uint32_t o = min(k0 + ks + 2 * i, p.K - 1) * kRowBytes;
+            __builtin_amdgcn_raw_buffer_store_b64(rec_u2_t{0u, 0u}, rsrc, o, 0, 0);
+#pragma unroll
+            for (int j = 0; j < CC; j += LD) {
+                if constexpr (LD == 4)
+                    __builtin_amdgcn_raw_buffer_store_b128(rec_u4_t{0u, 0u, 0u, 0u}, rsrc,
+                                                           o + 4u * (4 + c * CC + j), 0, 0);
+                else
+                    __builtin_amdgcn_raw_buffer_store_b64(rec_u2_t{0u, 0u}, rsrc,
+                                                          o + 4u * (4 + c * CC + j), 0, 0);
+            }
+        }
+    };
+    for (uint32_t k0 = 0;;) {
+        float mk[NS], Mc = -INFINITY;
+        bool vi[NS];
+#pragma unroll
+        for (int i = 0; i < NS; ++i) {
+            vi[i] = k0 + ks + 2 * i < k_live;
+            mk[i] = __uint_as_float(hw[i][0]) * kLog2e;
+            Mc = fmaxf(Mc, vi[i] ? mk[i] : -INFINITY);
+        }
+        if (k0 + 2 * NS >= k_live) zero_chunk(k0);
+        Mc = fmaxf(Mc, xor_lanes(Mc, 32));  // the other parity
+        const float Mn = fmaxf(M, Mc);
+        const float sc = M == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(M - Mn);
+        float lw = 0.0f;
+#pragma unroll
+        for (int j = 0; j < CC; ++j) a[j] *= sc;
+#pragma unroll
+        for (int i = 0; i < NS; ++i) {
+            const float w = vi[i] ? __builtin_amdgcn_exp2f(mk[i] - Mn) : 0.0f;
+            lw = fmaf(__uint_as_float(hw[i][1]), w, lw);
+#pragma unroll
+            for (int j = 0; j < CC; ++j) a[j] = fmaf(__uint_as_float(aw[i][j]), w, a[j]);
+        }
+        L = L * sc + (lw + xor_lanes(lw, 32));
+        M = Mn;
+        k0 += 2 * NS;
+        if (k0 >= k_live) break;
+        load_chunk(k0);
+    }
+    for (uint32_t k0 = 0; k0 + 2 * NS < k_live; k0 += 2 * NS) zero_chunk(k0);
+    // the two split parities
+#pragma unroll
+    for (int j = 0; j < CC; ++j) a[j] += xor_lanes(a[j], 32);
+    const float inv = L == 0.0f ? 0.0f : __builtin_amdgcn_rcpf(L);
+#pragma unroll
+    for (int j = 0; j < CC; ++j) v[j] = a[j] * inv;
+    egress_row<D>(v, es, gt, p.out + row * D, p.inv_sqrt_len, p.output_stage, lane);
+}
+
 __global__ void fill_zero_kernel(uint32_t* ptr, size_t words)
 {
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < words;
@@ -1556,6 +1662,26 @@ hipError_t launch_fused_t(hipStream_t stream, const DecodeParams& p, size_t lds)
                                lds_p, stream, p);
             return hipGetLastError();
         }
+    }
+    // Two launches where the combiner would be the long part: it merges its
+    // rows in one workgroup, four at a time, at a record round trip each, and
+    // reads and zeroes G x K x (d + 4) record words device-coherently on one
+    // CU; a launch of its own spreads the rows over all CUs for about 1.5 us
+    // more. Us fused / in two launches, K = 16 (K = 2): G = 16, d = 64 12.2 /
+    // 9.1 (15.0 / 11.6), d = 128 14.8 / 11.2 (17.2 / 14.8), d = 256 27.7 / 18.9
+    // (27.2 / 25.9); G = 8, d = 256 18.7 / 15.3, but 18.8 / 19.1 at K = 4, d =
+    // 128 10.1 / 9.7 and 9.7 / 10.0 at K = 8, d = 64 8.5 / 8.5; G = 4 and below
+    // loses or gains nothing. The test hooks are the fused wait's.
+    const bool hooks = p.withhold || p.poll_limit != kPollLimit;
+    const bool wide = p.G > 8 || (D == 256 && p.G > 4 && p.K >= 8);
+    if (p.K > 1 && wide && !hooks) {
+        hipLaunchKernelGGL((decode_kernel<D, 2, NS>), dim3((uint32_t)blocks), dim3(kThreads), lds,
+                           stream, p);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL((combine_live_kernel<D, NS>), dim3(p.B, (p.Hq + kWaves - 1) / kWaves),
+                           dim3(kThreads), 0, stream, p);
+        return hipGetLastError();
     }
     hipLaunchKernelGGL((decode_kernel<D, 1, NS>), dim3((uint32_t)blocks), dim3(kThreads), lds,
                        stream, p);

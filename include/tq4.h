@@ -212,6 +212,10 @@ int tq4_decode_poll_timeouts(void* stream, const void* workspace, size_t workspa
 /* Fused decode: partials, then one workgroup of each (seq, kv head) -- the
  * last of its splits to start -- waits for the others' records, LSE-combines
  * them in split order, rotates back, gates and stores BF16 -- one launch.
+ * (Wide GQA groups -- more than 8 q heads per kv head, more than 4 at
+ * head_size 256 with 8 splits or more -- whose grid fits the device combine in
+ * a second launch on the same stream instead, without tickets or waits; the
+ * workspace and its contract are the same.)
  * The wait is bounded and only on workgroups already running, so the launch
  * completes whatever the number of workgroups in flight.
  * Splits that hold no live token of their sequence (those at or past

@@ -569,15 +569,15 @@ def test_persistent_repeat_and_graph(tq4, oracle):
 
 @pytest.mark.parametrize("d", [64, 128, 256])
 @pytest.mark.parametrize("K", [2, 4, 5, 8, 9, 16])
-@pytest.mark.parametrize("B", [2, 160])
-def test_record_chunk_edges(tq4, oracle, d, K, B):
+@pytest.mark.parametrize("B,G", [(2, 4), (2, 8), (2, 16), (160, 3)])
+def test_record_chunk_edges(tq4, oracle, d, K, B, G):
     """Split counts at the edges of the combiner's record chunks (4, 8 and 16
-    splits), sequences with fewer live splits among them, a full and a partial
-    GQA group, the one-launch and the persistent kernel; the zeroed workspace
-    of one split count serves the next."""
+    splits), sequences with fewer live splits among them; the one-launch kernel
+    (G = 4), the two launches of wide groups and the persistent kernel; the
+    zeroed workspace of one split count serves the next."""
     import torch
-    rng = np.random.default_rng(1000 * d + 10 * K + B)
-    G, H, S = (16, 2, 16) if B == 2 else (3, 4, 16)
+    rng = np.random.default_rng(1000 * d + 10 * K + B + G)
+    H, S = (2, 16) if B == 2 else (4, 16)
     ctx = [int(x) for x in rng.integers(1, 16 * K + 1, B)]
     ctx[0] = 16 * K  # a page to a split, every split live
     P = sum((c + 15) // 16 for c in ctx) + 8
@@ -591,7 +591,7 @@ def test_record_chunk_edges(tq4, oracle, d, K, B):
     args = [dev(q), dev(kc), dev(vc), dev(sc), dev(tables), dev(ctx_a), dev(signs)]
     outs = [host(tq4.paged_decode(*args, H, S, P, workspace=ws, num_splits=k, scale=float(scale),
                                   inv_sqrt_len=float(isl))) for k in (K, 3, K)]
-    check_out(outs[0], want, f"record chunks d {d} K {K} B {B}")
+    check_out(outs[0], want, f"record chunks d {d} K {K} B {B} G {G}")
     assert np.array_equal(outs[0], outs[2])
     assert tq4.decode_poll_timeouts(ws, B, H) == 0
     assert not torch.any(ws)
@@ -613,3 +613,58 @@ def test_workspace_size_no_multiple_of_four(tq4, oracle):
                                   inv_sqrt_len=float(isl))) for w in (whole, odd, odd)]
     assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], outs[2])
     assert tq4.decode_poll_timeouts(odd, 1, H) == 0
+
+
+@pytest.mark.parametrize("d,G,K", [(64, 9, 40), (128, 16, 16), (256, 6, 8), (256, 16, 33)])
+@pytest.mark.parametrize("stage", [0, 1, 2])
+def test_wide_group_two_launches(tq4, oracle, d, G, K, stage):
+    """The decode of wide GQA groups in two launches: an empty sequence, one of
+    a single live split, one of every split, more splits than a record chunk,
+    the output stages; captured and replayed with eager calls of another split
+    count and of a narrow group on the same workspace in between."""
+    import torch
+    rng = np.random.default_rng(d + G + K + stage)
+    H, S = 2, 16
+    ctx = [K * 16, 0, 9, 16 * (K // 2) + 3, K * 16 - 1]
+    P = sum((c + 15) // 16 for c in ctx) + 4
+    kc, vc, sc, tables, signs, isl = build_cache(oracle, rng, ctx, H, d, S, P)
+    B, Hq = len(ctx), G * H
+    ctx_a = np.array(ctx, np.int32)
+    q = f32_to_bf16(rng.standard_normal((B, Hq, d)).astype(np.float32))
+    gate = rng.standard_normal((B, Hq, d)).astype(np.float32)
+    scale = np.float32(1.0 / math.sqrt(d))
+    _, want = oracle.paged_decode(q, kc, vc, sc, tables, ctx_a, signs, gate, Hq, H, d, S, P, K,
+                                  scale, isl, stage, threads=8)
+    ws = tq4.decode_workspace(B, Hq, H, d, K)
+    cache = [dev(x) for x in (kc, vc, sc, tables, ctx_a, signs)]
+    kw = dict(workspace=ws, scale=float(scale), inv_sqrt_len=float(isl), output_stage=stage)
+    dq, dg = dev(q), dev(gate)
+    out = torch.empty_like(dq)
+
+    def call():
+        tq4.paged_decode(dq, *cache, H, S, P, out=out, gate=dg, num_splits=K, **kw)
+
+    call()
+    first = host(out).copy()
+    check_out(first, want, f"wide group d {d} G {G} K {K} stage {stage}")
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call()
+    nq, ng = dq[:, :2 * H].contiguous(), dg[:, :2 * H].contiguous()
+    narrow = None
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(host(out), first)
+        tq4.paged_decode(dq, *cache, H, S, P, gate=dg, num_splits=3, **kw)
+        n = host(tq4.paged_decode(nq, *cache, H, S, P, gate=ng, num_splits=K // 2, **kw))
+        narrow = n if narrow is None else narrow
+        assert np.array_equal(n, narrow)
+    torch.cuda.synchronize()
+    assert not torch.any(ws)
