@@ -345,9 +345,9 @@ __global__ __launch_bounds__(kWriterThreads) void strip_writer(
 // the heads of a chunk, and the next head's rows are in flight under the
 // current head's arithmetic.
 // 8 ragged chunks of 17..2048 tokens (8256 tokens, 8 heads of 128):
-// 790 us a (request, head) item at a time, 18.0 us in chunks; bound there by
+// 790 us a (request, head) item at a time, 17.5 us in chunks; bound there by
 // the vector ALU (about 310 instructions a wave, chunk and head) and by the
-// chain of loads that a chunk begins with (lengths, slots, rows).
+// two loads in turn that a chunk begins with (slots, rows).
 
 // One lane's CPL consecutive BF16 channels as loaded (any alignment).
 template <int CPL>
@@ -432,7 +432,8 @@ __device__ __forceinline__ void store_key_word(int8_t* dst, const uint32_t (&t)[
 // Workgroups of the launch: as many as the registers keep resident on 256
 // CUs (four waves a SIMD, three at d = 256), so one generation takes it all.
 // 8 requests of 17..2048 tokens: 512 / 768 / 1024 / 2048 workgroups 18.7 /
-// 17.6 / 18.2 / 20.2 us; one of 8000 tokens 17.4 / 20.1 / 16.2 / 20.2 us.
+// 17.6 / 18.2 / 20.2 us; one of 8000 tokens 17.4 / 20.1 / 16.2 / 20.2 us
+// (both 0.5-0.7 us less since the requests' lengths and places are staged).
 template <int D>
 constexpr uint32_t kScatterGrid = D == 256 ? 768 : 1024;
 constexpr uint32_t kScatterPlan = 1024;  // requests whose chunk prefix is staged on chip
@@ -648,7 +649,12 @@ __global__ __launch_bounds__(kWriterThreads, D == 256 ? 3 : 4) void scatter_writ
     constexpr int CPL = D / 16;
     __shared__ __align__(16) uint32_t lds_t[2][D / 8][20];
     __shared__ __align__(16) int clash_w[kWriterThreads / 64];
-    __shared__ uint32_t chunks[kScatterPlan];  // inclusive prefix of the requests' chunks
+    // the requests: inclusive prefix of their chunks, first token, length, and
+    // the first token's place in its strip; read once here, so a chunk does not
+    // begin with two more dependent loads (the two cases above: 18.0 -> 17.5
+    // and 16.2 -> 15.5 us; 32 requests of 8 tokens 5.5 -> 5.2)
+    __shared__ uint32_t chunks[kScatterPlan], starts[kScatterPlan], counts[kScatterPlan];
+    __shared__ uint8_t places[kScatterPlan];
     const int tid = threadIdx.x, lane = tid & 63;
 
     if (probe != nullptr && blockIdx.x == 0 && tid < 32) {
@@ -670,14 +676,21 @@ __global__ __launch_bounds__(kWriterThreads, D == 256 ? 3 : 4) void scatter_writ
             for (uint32_t b = 0; b < nr; b += 64) {
                 const uint32_t i = min(b + lane, nr - 1);
                 const uint32_t t0 = (uint32_t)cu[i], t1 = (uint32_t)cu[i + 1];
-                uint32_t v = b + lane < nr && t1 > t0 ? (t1 - t0 + 30u) >> 4 : 0u;
+                const uint32_t n = t1 > t0 ? t1 - t0 : 0u;
+                const int32_t s0 = n > 0 ? p.slots[t0] : -1;
+                uint32_t v = b + lane < nr && n > 0 ? (n + 30u) >> 4 : 0u;
 #pragma unroll
                 for (int o = 1; o < 64; o <<= 1) {
                     const uint32_t w = __shfl_up(v, o, 64);
                     if (lane >= o) v += w;
                 }
                 v += carry;
-                if (b + lane < nr) chunks[i] = v;
+                if (b + lane < nr) {
+                    chunks[i] = v;
+                    starts[i] = t0;
+                    counts[i] = n;
+                    places[i] = s0 >= 0 ? s0 % kStrip : 0;
+                }
                 carry = __shfl(v, 63, 64);
             }
         }
@@ -700,13 +713,15 @@ __global__ __launch_bounds__(kWriterThreads, D == 256 ? 3 : 4) void scatter_writ
         i = __builtin_amdgcn_readfirstlane(i);
         for (uint64_t left = per; left > 0 && i < nr;) {
             const uint32_t take = (uint32_t)min(left, (uint64_t)(p.H - h));
-            const uint32_t c = v - (i > 0 ? chunks[i - 1] : 0u);
+            const uint32_t c =
+                v - (i > 0 ? __builtin_amdgcn_readfirstlane(chunks[i - 1]) : 0u);
             const uint64_t item0 = (rb + i) * p.H;  // the request's heads inside the window
             const uint32_t h0 = (uint32_t)(max(item0 + h, (uint64_t)item_begin) - item0);
             const uint32_t h1 = (uint32_t)(min(item0 + h + take, item_end) - item0);
-            const uint32_t t0 = (uint32_t)cu[i], n = (uint32_t)cu[i + 1] - t0;
-            const int32_t s0 = p.slots[t0];
-            const int64_t first = (int64_t)c * kStrip - (s0 >= 0 ? s0 % kStrip : 0);
+            const uint32_t t0 = __builtin_amdgcn_readfirstlane(starts[i]);
+            const uint32_t n = __builtin_amdgcn_readfirstlane(counts[i]);
+            const int64_t first =
+                (int64_t)c * kStrip - __builtin_amdgcn_readfirstlane((int)places[i]);
             if ((int32_t)(h1 - h0) > 0 && first < (int64_t)n) {
                 if (!scatter_chunk<D>(p, t0, n, first, h0, h1, sign, lds_t, clash_w))
                     scatter_tokens<D>(p, t0, n, first, h0, h1, sign);
