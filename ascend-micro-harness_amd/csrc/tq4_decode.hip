@@ -761,6 +761,20 @@ __device__ __forceinline__ void build_qops(QOps<D>& qo, const float* q_st, const
     qo.bias4 = f4_t{bias, bias, bias, bias};
 }
 
+// Place of the parked rows' float4 e4 = row * d/4 + channel / 4. A lane holds
+// d/16 consecutive channels, so in order the 16 lanes of a row would store
+// each of their float4s d/64 quads apart: on 16 / (d/64) of the 16 bank quads.
+// The bits of e4 above 4 spread them over all; 16 consecutive float4s stay
+// within one aligned group of 16 or fewer, so the readers' order costs nothing.
+// In order, parking 16 rows of 256 took 3.0 us of a split (0.8 us for 4 rows);
+// 64 splits of 256 tokens at 16 heads of 256 16.8 -> 14.1 us (the combine
+// included), of 128 10.2 -> 9.7, 4 heads of 256 12.2 -> 11.9, of 128 the same.
+template <int D>
+__device__ __forceinline__ uint32_t part_quad(uint32_t e4)
+{
+    return e4 ^ ((e4 >> 4) & (D / 64 - 1));
+}
+
 // Park one wave's rows for the merge: (m, l, 2^-sh) per row at [row][wave]
 // (one 16-byte read gives a row's four waves), with EXACT the row's exact
 // maximum score at t_x, and the raw rows (offset column removed) at part
@@ -786,9 +800,13 @@ __device__ __forceinline__ void park_rows(const RowState<D>& st, bool row_live, 
     for (int i = 0; i < 4; ++i) {
         const uint32_t r = 4 * g4 + i;
         if (r < G) {
-            float* dst = part + ((size_t)wave * G + r) * D + n * NB;  // channel n*d/16 + b
+            // channel n*d/16 + b
+            float* dst = part + (size_t)wave * G * D;
 #pragma unroll
-            for (int b = 0; b < NB; ++b) dst[b] = st.acc[b][i] - st.cr[i];
+            for (int b = 0; b < NB; b += 4)
+                *(float4*)(dst + 4 * part_quad<D>((r * D + n * NB + b) / 4)) =
+                    make_float4(st.acc[b][i] - st.cr[i], st.acc[b + 1][i] - st.cr[i],
+                                st.acc[b + 2][i] - st.cr[i], st.acc[b + 3][i] - st.cr[i]);
         }
     }
 }
@@ -865,7 +883,7 @@ __device__ __forceinline__ void finish_item(const DecodeParams& p, uint32_t seq,
         float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll
         for (int w = 0; w < kWaves; ++w) {
-            const float4 x = *(const float4*)(part + (size_t)w * G * D + 4 * e4);
+            const float4 x = *(const float4*)(part + (size_t)w * G * D + 4 * part_quad<D>(e4));
             const float fw = f[w] * kValueUnit;
             v.x += x.x * fw;
             v.y += x.y * fw;
@@ -985,7 +1003,7 @@ __device__ __forceinline__ void finish_item(const DecodeParams& p, uint32_t seq,
             const float inv = L == 0.0f ? 0.0f : 1.0f / L;
             v = L == 0.0f ? make_float4(0.0f, 0.0f, 0.0f, 0.0f)
                           : make_float4(v.x * inv, v.y * inv, v.z * inv, v.w * inv);
-            *(float4*)(part + 4 * e4) = v;
+            *(float4*)(part + 4 * part_quad<D>(e4)) = v;
         }
         lds_barrier();
         for (uint32_t g = wave; g < G; g += kWaves) {
@@ -994,7 +1012,10 @@ __device__ __forceinline__ void finish_item(const DecodeParams& p, uint32_t seq,
             if (p.output_stage == 2) load_lane_floats<D>(p.gate + qh * D, lane, gt);
             float v[CC];
 #pragma unroll
-            for (int j = 0; j < CC; ++j) v[j] = part[g * D + (lane & 31) * CC + j];
+            for (int j = 0; j < CC; ++j) {
+                const uint32_t e = g * D + (lane & 31) * CC + j;
+                v[j] = part[4 * part_quad<D>(e / 4) + e % 4];
+            }
             egress_row<D>(v, es, gt, p.out + qh * D, p.inv_sqrt_len, p.output_stage, lane);
         }
     }
