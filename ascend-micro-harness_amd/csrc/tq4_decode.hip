@@ -366,7 +366,9 @@ __device__ void combine_records(const float* rr, uint32_t K, int lane, float (&v
             Mc = fmaxf(Mc, vi[i] ? mk[i] : -INFINITY);
         }
         Mc = fmaxf(Mc, xor_lanes(Mc, 32));  // the other parity
-        const float Mn = fmaxf(M, Mc);
+        // Held at kMasked: in log2 units a neutral record's maximum overflows to
+        // -inf, and under a maximum of -inf too its weight would be a NaN.
+        const float Mn = fmaxf(fmaxf(M, Mc), kMasked);
         const float sc = M == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(M - Mn);
         float lw = 0.0f;
 #pragma unroll
@@ -1620,7 +1622,7 @@ __global__ __launch_bounds__(kThreads) void combine_live_kernel(DecodeParams p)
         }
         if (k0 + 2 * NS >= k_live) zero_chunk(k0);
         Mc = fmaxf(Mc, xor_lanes(Mc, 32));  // the other parity
-        const float Mn = fmaxf(M, Mc);
+        const float Mn = fmaxf(fmaxf(M, Mc), kMasked);  // as combine_records
         const float sc = M == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(M - Mn);
         float lw = 0.0f;
 #pragma unroll
