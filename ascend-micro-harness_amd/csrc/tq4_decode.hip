@@ -248,6 +248,52 @@ __device__ __forceinline__ void load_row_chunk(uint32_t (&k)[D / 32], const int8
 }
 
 
+// One chunk of records (decoded by ^ x) into a row's running maximum, sum and
+// accumulators. vi: the slots that hold a split; full: all of them do
+// (wave-uniform). A slot that holds none repeats another record, which may be
+// infinite, so it is selected out, never weighted 0.
+template <int NS, int CC>
+__device__ __forceinline__ void combine_chunk(const uint32_t (&hw)[NS][2],
+                                              const uint32_t (&aw)[NS][CC], const bool (&vi)[NS],
+                                              bool full, uint32_t x, float& M, float& L,
+                                              float (&a)[CC])
+{
+    float mk[NS], Mc = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+        mk[i] = __uint_as_float(hw[i][0] ^ x) * kLog2e;
+        Mc = fmaxf(Mc, vi[i] ? mk[i] : -INFINITY);
+    }
+    Mc = fmaxf(Mc, xor_lanes(Mc, 32));  // the other parity
+    // Held at kMasked: in log2 units a neutral record's maximum overflows to
+    // -inf, and under a maximum of -inf too its weight would be a NaN.
+    const float Mn = fmaxf(fmaxf(M, Mc), kMasked);
+    const float sc = M == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(M - Mn);
+    float lw = 0.0f;
+#pragma unroll
+    for (int j = 0; j < CC; ++j) a[j] *= sc;
+    if (full) {
+        // one decode and one fma per word, no select
+#pragma unroll
+        for (int i = 0; i < NS; ++i) {
+            const float w = __builtin_amdgcn_exp2f(mk[i] - Mn);
+            lw = fmaf(__uint_as_float(hw[i][1] ^ x), w, lw);
+#pragma unroll
+            for (int j = 0; j < CC; ++j) a[j] = fmaf(__uint_as_float(aw[i][j] ^ x), w, a[j]);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < NS; ++i) {
+            const float w = __builtin_amdgcn_exp2f(mk[i] - Mn);
+            lw += vi[i] ? __uint_as_float(hw[i][1] ^ x) * w : 0.0f;
+#pragma unroll
+            for (int j = 0; j < CC; ++j) a[j] += vi[i] ? __uint_as_float(aw[i][j] ^ x) * w : 0.0f;
+        }
+    }
+    L = L * sc + (lw + xor_lanes(lw, 32));
+    M = Mn;
+}
+
 // Combine layout of one wave over one (seq, q head) row: lane c = lane & 31
 // owns channels c*CC .. c*CC+CC-1 (CC = d/32); ks = lane >> 5 takes the
 // splits of parity ks of every round of 2*NS, so a round costs each lane NS
@@ -359,42 +405,7 @@ __device__ void combine_records(const float* rr, uint32_t K, int lane, float (&v
         if constexpr (FUSED) {
             if (k0 + 2 * NS >= K) zero_chunk(k0);
         }
-        float mk[NS], Mc = -INFINITY;
-#pragma unroll
-        for (int i = 0; i < NS; ++i) {
-            mk[i] = __uint_as_float(hw[i][0] ^ x) * kLog2e;
-            Mc = fmaxf(Mc, vi[i] ? mk[i] : -INFINITY);
-        }
-        Mc = fmaxf(Mc, xor_lanes(Mc, 32));  // the other parity
-        // Held at kMasked: in log2 units a neutral record's maximum overflows to
-        // -inf, and under a maximum of -inf too its weight would be a NaN.
-        const float Mn = fmaxf(fmaxf(M, Mc), kMasked);
-        const float sc = M == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(M - Mn);
-        float lw = 0.0f;
-#pragma unroll
-        for (int j = 0; j < CC; ++j) a[j] *= sc;
-        if (k0 + 2 * NS <= K) {
-            // every slot of the chunk holds a split (wave-uniform): one
-            // decode and one fma per word, no select
-#pragma unroll
-            for (int i = 0; i < NS; ++i) {
-                const float w = __builtin_amdgcn_exp2f(mk[i] - Mn);
-                lw = fmaf(__uint_as_float(hw[i][1] ^ x), w, lw);
-#pragma unroll
-                for (int j = 0; j < CC; ++j) a[j] = fmaf(__uint_as_float(aw[i][j] ^ x), w, a[j]);
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < NS; ++i) {
-                const float w = __builtin_amdgcn_exp2f(mk[i] - Mn);
-                lw += vi[i] ? __uint_as_float(hw[i][1] ^ x) * w : 0.0f;
-#pragma unroll
-                for (int j = 0; j < CC; ++j)
-                    a[j] += vi[i] ? __uint_as_float(aw[i][j] ^ x) * w : 0.0f;
-            }
-        }
-        L = L * sc + (lw + xor_lanes(lw, 32));
-        M = Mn;
+        combine_chunk<NS, CC>(hw, aw, vi, k0 + 2 * NS <= K, x, M, L, a);
     }
     if constexpr (FUSED) {
         for (uint32_t k0 = 0; k0 + 2 * NS < K; k0 += 2 * NS) zero_chunk(k0);
@@ -1548,7 +1559,8 @@ __global__ __launch_bounds__(kThreads) void combine_kernel(DecodeParams p)
 
 // The second of the fused decode's two launches: one (seq, q head) row per
 // wave over the records of the sequence's live splits (the layout, the order
-// and the arithmetic of combine_records), zeroed once read. The first chunk's
+// and the arithmetic of combine_records, by the same combine_chunk), zeroed
+// once read. The first chunk's
 // loads do not wait for the context length that says which splits are live:
 // the records of dead ones are in range and all zero, and are selected out.
 // Rows of one live split (or none) are finished by the first launch.
@@ -1612,30 +1624,11 @@ __global__ __launch_bounds__(kThreads) void combine_live_kernel(DecodeParams p)
         }
     };
     for (uint32_t k0 = 0;;) {
-        float mk[NS], Mc = -INFINITY;
         bool vi[NS];
 #pragma unroll
-        for (int i = 0; i < NS; ++i) {
-            vi[i] = k0 + ks + 2 * i < k_live;
-            mk[i] = __uint_as_float(hw[i][0]) * kLog2e;
-            Mc = fmaxf(Mc, vi[i] ? mk[i] : -INFINITY);
-        }
+        for (int i = 0; i < NS; ++i) vi[i] = k0 + ks + 2 * i < k_live;
         if (k0 + 2 * NS >= k_live) zero_chunk(k0);
-        Mc = fmaxf(Mc, xor_lanes(Mc, 32));  // the other parity
-        const float Mn = fmaxf(fmaxf(M, Mc), kMasked);  // as combine_records
-        const float sc = M == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(M - Mn);
-        float lw = 0.0f;
-#pragma unroll
-        for (int j = 0; j < CC; ++j) a[j] *= sc;
-#pragma unroll
-        for (int i = 0; i < NS; ++i) {
-            const float w = vi[i] ? __builtin_amdgcn_exp2f(mk[i] - Mn) : 0.0f;
-            lw = fmaf(__uint_as_float(hw[i][1]), w, lw);
-#pragma unroll
-            for (int j = 0; j < CC; ++j) a[j] = fmaf(__uint_as_float(aw[i][j]), w, a[j]);
-        }
-        L = L * sc + (lw + xor_lanes(lw, 32));
-        M = Mn;
+        combine_chunk<NS, CC>(hw, aw, vi, k0 + 2 * NS <= k_live, 0u, M, L, a);
         k0 += 2 * NS;
         if (k0 >= k_live) break;
         load_chunk(k0);

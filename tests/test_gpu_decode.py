@@ -668,3 +668,29 @@ def test_wide_group_two_launches(tq4, oracle, d, G, K, stage):
         assert np.array_equal(n, narrow)
     torch.cuda.synchronize()
     assert not torch.any(ws)
+
+
+@pytest.mark.parametrize("d,K", [(64, 3), (128, 3), (128, 5), (256, 9)])
+def test_wide_group_infinite_record(tq4, d, K):
+    """A record whose accumulators overflow to infinity, in the last split (8192
+    equal scores over values of 7 * 2^113): the combine launch of a wide group
+    gives what the one-launch kernel gives for the same query heads in narrow
+    groups, infinities of the values' signs and no NaN."""
+    H, S, G, n = 1, 128, 16, 64  # n pages a split
+    P = n * K
+    kc = np.zeros(P * H * S * d // 2, np.int8)
+    sign = np.where(np.arange(d) % 3 == 0, -1.0, 1.0)
+    vc = np.where(sign < 0, -0x67, 0x77).astype(np.int8)  # codes -7, -7 and 7, 7
+    vc = np.tile(np.repeat(vc, 8), P * H * S // 16)       # a channel's 16 tokens
+    sc = np.ones(2 * P * H * S, np.float32)
+    sc[(P + n * (K - 1)) * H * S:] = 2.0 ** 113
+    cache = [dev(x) for x in (kc, vc, sc, np.arange(P, dtype=np.int32)[None, :],
+                              np.array([P * S], np.int32), np.ones(d, np.float32))]
+
+    def call(heads):
+        return host(tq4.paged_decode(dev(np.zeros((1, heads, d), np.uint16)), *cache, H, S, P,
+                                     num_splits=K, output_stage=0))
+
+    wide, narrow = call(G), call(4)
+    assert np.array_equal(bf16_to_f32(narrow), np.broadcast_to(sign * np.inf, (1, 4, d)))
+    assert np.array_equal(wide, np.tile(narrow, (1, 4, 1)))
