@@ -240,30 +240,46 @@ uint32_t tq4_decode_auto_splits_lens(uint32_t num_seqs, uint32_t num_kv_heads,
         sum += c;
         if (c > mx) mx = c;
     }
-    // Unless one sequence is several times the mean, workgroups that fill the
-    // CUs are not split again: a second wave of shorter items costs more than
-    // it evens out. Us with / without the second split, lengths spread over
-    // half to the whole of the longest: 4 sequences x 8 KV heads at ctx 12000
-    // 16.1 / 13.0 (d = 256 35.3 / 22.3), 8 at 12000 20.9 / 18.1 (46.8 / 36.4),
-    // 16 at 4096 15.3 / 14.6 (36.3 / 28.7), 32 at 2048 17.4 / 15.5 (44.8 /
-    // 31.8); 12 sequences (fill 3/4) still want it: 26.6 against 29.1.
-    uint32_t k = split_rule(num_seqs, num_kv_heads, max_blocks_per_seq, block_size,
-                            mx * num_seqs < 3 * sum);
-    // A ragged batch (longest context >= 1.6 x the mean) whose (seq, kv head)
-    // items fill the resident slots (512 at d <= 128) between half and one
-    // and a half times: one item per (seq, kv head) leaves the launch waiting
-    // on the longest sequences, so split them at least three ways, four when
-    // a longest item alone fills its CU. Measured (64 x U[512, 8192]: 75.4 ->
-    // 72.3 us; 64 x U[128, 16384]: 133.3 -> 125.2; 80 x U[512, 8192]: 96.5 ->
-    // 92.7; 32 x U[1200, 12000]: 58.1 -> 52.9), while a uniform or mildly
-    // ragged batch (64 x 8192, 64 x U[2048, 8192]) and short contexts (40 x
-    // U[100, 1024]: 12.9 against 17.3) run best as they are.
+    // Workgroups that fill the CUs are not split again unless the lengths are
+    // skewed: a second wave of shorter items costs more than it evens out. Us
+    // with / without the second split, lengths spread over half to the whole
+    // of the longest: 4 sequences x 8 KV heads at ctx 12000 16.1 / 13.0 (d =
+    // 256 35.3 / 22.3), 8 at 12000 20.9 / 18.1 (46.8 / 36.4), 16 at 4096 15.3 /
+    // 14.6 (36.3 / 28.7), 32 at 2048 17.4 / 15.5 (44.8 / 31.8); 12 sequences
+    // (fill 3/4) still want it: 26.6 against 29.1. Up to 256 items the line
+    // lies at a longest of 15/8 the mean (30 x 4 KV heads at 2.9 x the mean, d =
+    // 64, ctx 22681: 24.3 / 37.0; 15 x 4 at 2.7 x, d = 256, 11722: 23.0 / 29.7;
+    // over 160 batches of 16 to 300 items the former line at 3 x lost up to a
+    // third, this one 3 %), past them at 3 x.
     const uint64_t items = (uint64_t)num_seqs * num_kv_heads;
-    const bool ragged = sum > 0 && mx * num_seqs * 5 >= sum * 8;
-    const uint32_t want = items > 256 && items <= 768 && mx >= 192 * kStrip    ? 3
-                          : items > 192 && items <= 256 && mx >= 512 * kStrip ? 4
-                                                                              : 1;
-    if (ragged && k < want && max_blocks_per_seq >= want) k = want;
+    const uint64_t top = mx * num_seqs;
+    uint32_t k = split_rule(num_seqs, num_kv_heads, max_blocks_per_seq, block_size,
+                            items <= 256 ? top * 8 < sum * 15 : top < sum * 3);
+    // A ragged batch whose (seq, kv head) items fill the resident slots (512 at
+    // d <= 128) between half and one and a half times: one item per (seq, kv
+    // head) leaves the launch waiting on the longest sequences, so split them
+    // at least three ways. Measured (64 x 8 x U[512, 8192]: 75.4 -> 72.3 us; 64
+    // x U[128, 16384]: 133.3 -> 125.2; 80 x U[512, 8192]: 96.5 -> 92.7), while
+    // a uniform or mildly ragged batch (64 x 8192, 64 x U[2048, 8192]) and short
+    // contexts (40 x U[100, 1024]: 12.9 against 17.3) run best as they are. Of
+    // the short ones, two splits lose to three where one sequence is several
+    // times the mean (42 x 8 at 6.5 x, ctx 1744: 13.0 / 12.0; 372 items at 4.9 x,
+    // d = 256, ctx 2972: 34.9 / 32.2).
+    // 193 to 256 items whose longest alone fills a CU (512 strips): three, four
+    // where they fill the CUs' slots in whole rounds (256 items) or one sequence
+    // is 3 times the mean. 256 items, 60 batches at d = 64, 128 and 256: four
+    // against two 1.12 times as fast in the middle (r >= 7/4 the mean; below it
+    // loses at d = 64); fewer items: four against three 0.92 to 1.07 below 3 x
+    // the mean, 1.04 to 1.19 from there.
+    uint32_t want = 1;
+    if (sum > 0 && top * 5 >= sum * 8) {
+        if (items > 256 && items <= 768) {
+            if (mx >= 192 * kStrip || (k == 2 && top * 2 >= sum * 7)) want = 3;
+        } else if (items > 192 && items <= 256 && mx >= 512 * kStrip && top * 4 >= sum * 7) {
+            want = items == 256 || top >= sum * 3 ? 4 : 3;
+        }
+    }
+    if (k < want && max_blocks_per_seq >= want) k = want;
     return k;
 }
 

@@ -178,22 +178,25 @@ size_t tq4_decode_workspace_bytes(uint32_t num_seqs, uint32_t num_heads, uint32_
 uint32_t tq4_decode_auto_splits(uint32_t num_seqs, uint32_t num_kv_heads,
                                 uint32_t max_blocks_per_seq, uint32_t block_size);
 
+/* tq4_decode_auto_splits for a caller that holds the context lengths on the
+ * host (context_lens: num_seqs host integers; NULL gives the plain rule). A
+ * batch whose workgroups fill the CUs is not split further unless its longest
+ * context is 15/8 the mean (3 times, past 256 (seq, kv head) items). A ragged
+ * batch (longest >= 1.6 x mean) of 257 to 768 items takes at least 3 splits
+ * when its longest context has 192 strips, one of 193 to 256 items (>= 7/4 x
+ * mean) 3 or 4 from 512 strips on. The count is chosen for speed alone: with
+ * 256 items of 16 heads of 256 its records pass the 16 MiB of
+ * tq4_paged_decode_noalloc. No reference counterpart (the reference's callers
+ * pass their split count). */
+uint32_t tq4_decode_auto_splits_lens(uint32_t num_seqs, uint32_t num_kv_heads,
+                                     uint32_t max_blocks_per_seq, uint32_t block_size,
+                                     const int32_t* context_lens);
+
 /* Zero a workspace (a fill kernel, no memset node). The fused entry needs a
  * zeroed workspace before its first call and leaves it zeroed after every
  * call (its counters, and its records, which it consumes and clears); a
  * workspace that tq4_paged_decode_partials has written since must be zeroed
  * again before tq4_paged_decode uses it. */
-/* tq4_decode_auto_splits for a caller that holds the context lengths on the
- * host (context_lens: num_seqs host integers; NULL gives the plain rule).
- * Unless the longest is 3 times the mean, a batch whose workgroups fill the
- * CUs is not split further; a ragged batch (longest >= 1.6 x mean) of 257 to
- * 768 (seq, kv head) items takes at least 3 splits when its longest context
- * has 192 strips, one of 193 to 256 items at least 4 from 512 strips on. No
- * reference counterpart (the reference's callers pass their split count). */
-uint32_t tq4_decode_auto_splits_lens(uint32_t num_seqs, uint32_t num_kv_heads,
-                                     uint32_t max_blocks_per_seq, uint32_t block_size,
-                                     const int32_t* context_lens);
-
 int tq4_decode_workspace_init(void* stream, void* workspace, size_t workspace_bytes);
 
 /* The fused entry's timeout count: rows (times 16-split record chunks) whose

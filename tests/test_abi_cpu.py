@@ -335,3 +335,24 @@ def test_auto_splits_short_filled_and_ragged(lib):
     assert lens(64, 64, [16 * (i + 1) for i in range(64)]) == 1
     for mb, page in ((8192, 16), (70000, 16), (3, 1024)):  # the staged window's bound
         assert -(-mb // f(1, 1, mb, page)) * (page // 16) <= 2048
+
+
+def test_auto_splits_skewed_lengths(lib):
+    """Batches whose longest context is two to three times the mean are split
+    past the CUs up to 256 (seq, kv head) items; short skewed batches of 257 to
+    768 items take three splits or one, not two; the 193 to 256 item rule."""
+    import numpy as np
+    g = lib.tq4_decode_auto_splits_lens
+    g.restype = C.c_uint32
+    g.argtypes = [C.c_uint32] * 4 + [C.c_void_p]
+
+    def power(n, H, hi, e, page=16):  # longest = about e + 1 times the mean
+        a = np.array([max(1, int(hi * ((i + 1) / n) ** e)) for i in range(n)], np.int32)
+        return g(n, H, -(-hi // page), page, a.ctypes.data)
+
+    assert power(30, 4, 22681, 2) == 5 and power(15, 4, 11722, 2) == 9
+    assert power(30, 4, 22681, 0.33) == 3 and power(15, 4, 11722, 0.33) == 4
+    assert power(42, 8, 1744, 6) == 3 and power(186, 2, 2972, 4) == 3  # several x the mean
+    assert power(60, 8, 1744, 1) == 1 and power(42, 8, 900, 6) == 1
+    assert power(106, 2, 13818, 1.5) == 3 and power(106, 2, 13818, 4) == 4
+    assert power(32, 8, 12129, 1.3) == 4 and power(128, 2, 16117, 0.55) == 2
