@@ -334,20 +334,32 @@ __global__ __launch_bounds__(kWriterThreads) void strip_writer(
 //     other token of the request touches is written at once (scatter_chunk):
 //     the strip writer's arithmetic and transpose, the value strip's words
 //     merged under the mask of the columns written (whole words are stored
-//     without a read). To know that no other token touches the strip, the
-//     workgroup reads the request's slots (4 bytes a token against the
-//     5 x head_size bytes a head of the token costs) under its rows' loads.
+//     without a read).
+//   * To know that no other token touches the strip, a chunk of a request of
+//     up to 8192 tokens reads the request's slots under its rows' loads (32 KB
+//     a chunk there, from the caches). That grows with the square of the length,
+//     so of longer requests a workgroup searches the chunks of its run together,
+//     16 to a pass over the slots (scatter_search); a request of one chunk
+//     needs no search.
 //   * Any other chunk goes token by token (scatter_tokens): a strip belongs to
 //     the chunk that holds its first token, which writes all of its tokens in
 //     token order; the other chunks skip them. So one workgroup at a time
-//     merges into a strip, and of two tokens with one slot the later wins.
+//     merges into a strip, and of two tokens with one slot the later wins. It
+//     reads the request's slots once a token, so a fully shuffled request
+//     costs the square of its length (8192 tokens x 8 heads: 1.0 ms; 18.4 ms
+//     item by item).
 // A workgroup takes a run of (chunk, head) pairs: the slots are read once for
 // the heads of a chunk, and the next head's rows are in flight under the
 // current head's arithmetic.
 // 8 ragged chunks of 17..2048 tokens (8256 tokens, 8 heads of 128):
-// 790 us a (request, head) item at a time, 17.5 us in chunks; bound there by
+// 790 us a (request, head) item at a time, 16.8 us in chunks; bound there by
 // the vector ALU (about 310 instructions a wave, chunk and head) and by the
-// two loads in turn that a chunk begins with (slots, rows).
+// two loads in turn that a chunk begins with (slots, rows). One request of
+// 32768 / 131072 tokens, 8 heads of 128: 66 / 465 us with a search a chunk,
+// 56 / 230 together (64 requests of 2048: 169). Requests of one token, 8 heads
+// (1 head): 256 of them 9.5 (5.2) us, 1024 22.9 (8.2), 4096 77 (23.5); item by
+// item 9.3 (4.6), 27.9 (6.2) and 98 (15.7): there the one head's workgroups
+// wait for the chunk count that a workgroup to an item does without.
 
 // One lane's CPL consecutive BF16 channels as loaded (any alignment).
 template <int CPL>
@@ -433,10 +445,26 @@ __device__ __forceinline__ void store_key_word(int8_t* dst, const uint32_t (&t)[
 // CUs (four waves a SIMD, three at d = 256), so one generation takes it all.
 // 8 requests of 17..2048 tokens: 512 / 768 / 1024 / 2048 workgroups 18.7 /
 // 17.6 / 18.2 / 20.2 us; one of 8000 tokens 17.4 / 20.1 / 16.2 / 20.2 us
-// (both 0.5-0.7 us less since the requests' lengths and places are staged).
+// (1024 at 16.8 and 15.5 since the requests' lengths and places are staged).
 template <int D>
 constexpr uint32_t kScatterGrid = D == 256 ? 768 : 1024;
 constexpr uint32_t kScatterPlan = 1024;  // requests whose chunk prefix is staged on chip
+
+// The search for other tokens in the strips of a run's chunks (scatter_search).
+constexpr uint32_t kGroup = kWriterThreads / kStrip;  // chunks to a pass: a slot a thread
+constexpr uint32_t kTable = kWriterThreads;           // their strips, open-addressed
+constexpr int32_t kNoStrip = 0x7fffffff;              // above every slot / 16
+// Longer requests are searched by runs: a pass of its own costs more than the
+// search under the rows' loads until the run has several chunks (8 heads: 8192
+// tokens 20.9 us a chunk at a time, 21.5 together; 32768 66 / 56).
+constexpr uint32_t kSearchFrom = 8192;
+constexpr uint32_t kSearchRun = 256;  // chunks of a run searched together at most
+struct SearchShared {
+    int32_t table[kTable];
+    uint32_t owner[kTable];
+    uint32_t clash;
+    uint8_t found[kSearchRun];  // the run's chunks (modulo its size) with a clash
+};
 
 struct ScatterArgs {
     const uint16_t *key, *value;
@@ -474,52 +502,125 @@ __device__ __forceinline__ void scatter_tokens(const ScatterArgs& p, uint32_t t0
         if (!slot_in_pool(slot0, p.S, p.P)) continue;
         const int32_t strip = slot0 >> 4;
         int seen = 0;  // an earlier token of the request in this strip
-        for (uint32_t u = tid; u < i0; u += kWriterThreads) seen |= (p.slots[t0 + u] >> 4) == strip;
-        if (__syncthreads_or(seen)) continue;
-        for (uint32_t base = i0; base < n; base += 64) {
-            const uint32_t u = base + (tid & 63);
-            const bool in = u < n && (p.slots[t0 + u] >> 4) == strip;
-            for (uint64_t m = __ballot(in); m != 0; m &= m - 1) {
-                const uint32_t token = t0 + base + (uint32_t)__builtin_ctzll(m);
-                const uint32_t slot = (uint32_t)p.slots[token];
-                const uint32_t page = slot / p.S, tip = slot % p.S, col = tip % kStrip;
-                for (uint32_t h = h0 + (tid >> 4); h < h1; h += kWriterThreads / 16) {
-                    const size_t src = ((size_t)token * p.H + h) * D + l * CPL;
-                    RawRow<CPL> rk, rv;
-                    load_raw<CPL>(p.key + src, rk);
-                    load_raw<CPL>(p.value + src, rv);
-                    float v[2][CPL], a[2], sc[2];
-                    unpack_raw<CPL>(rk, v[0]);
-                    unpack_raw<CPL>(rv, v[1]);
-                    writer_rotate<D, CPL>(v, sign, l);
-                    writer_absmax<CPL>(v, 0.0f, a);
-                    uint32_t t[2][CPL];
-                    quantise_exact<CPL>(v, a, sigma, p.inv_sqrt_len, t, sc);
-                    const size_t row = ((size_t)page * p.H + h) * p.S + tip;
-                    if ((tid & 15) == 0) {
-                        p.scale_cache[row] = sc[0];
-                        p.scale_cache[(size_t)p.P * p.H * p.S + row] = sc[1];
-                    }
-                    store_key_word<CPL>(p.key_cache + row * (D / 2) + l * (CPL / 2), t[0]);
-                    uint32_t* words = (uint32_t*)(p.value_cache + (row - col) * (D / 2)) +
-                                      2 * l * CPL + (col >> 3);
-                    const uint32_t sh = 4u * (col & 7u);
+        const int32_t* sl = p.slots + t0;
+        for (uint32_t u = tid; u < i0; u += 4 * kWriterThreads) {
 #pragma unroll
-                    for (int j = 0; j < CPL; ++j)
-                        words[2 * j] = (words[2 * j] & ~(0xfu << sh)) |
-                                       (((t[1][j] ^ 8u) & 0xfu) << sh);
+            for (int k = 0; k < 4; ++k) seen |= (sl[min(u + k * kWriterThreads, i0 - 1)] >> 4) == strip;
+        }
+        if (__syncthreads_or(seen)) continue;
+        for (uint32_t base = i0; base < n; base += 4 * 64) {
+            uint64_t in[4];  // four loads in flight
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const uint32_t u = base + 64 * k + (tid & 63);
+                in[k] = __ballot((sl[min(u, n - 1)] >> 4) == strip && u < n);
+            }
+#pragma unroll 1
+            for (int k = 0; k < 4; ++k) {
+                uint64_t m = k == 0 ? in[0] : k == 1 ? in[1] : k == 2 ? in[2] : in[3];
+                for (; m != 0; m &= m - 1) {
+                    const uint32_t token = t0 + base + 64 * k + (uint32_t)__builtin_ctzll(m);
+                    const uint32_t slot = (uint32_t)p.slots[token];
+                    const uint32_t page = slot / p.S, tip = slot % p.S, col = tip % kStrip;
+                    for (uint32_t h = h0 + (tid >> 4); h < h1; h += kWriterThreads / 16) {
+                        const size_t src = ((size_t)token * p.H + h) * D + l * CPL;
+                        RawRow<CPL> rk, rv;
+                        load_raw<CPL>(p.key + src, rk);
+                        load_raw<CPL>(p.value + src, rv);
+                        float v[2][CPL], a[2], sc[2];
+                        unpack_raw<CPL>(rk, v[0]);
+                        unpack_raw<CPL>(rv, v[1]);
+                        writer_rotate<D, CPL>(v, sign, l);
+                        writer_absmax<CPL>(v, 0.0f, a);
+                        uint32_t t[2][CPL];
+                        quantise_exact<CPL>(v, a, sigma, p.inv_sqrt_len, t, sc);
+                        const size_t row = ((size_t)page * p.H + h) * p.S + tip;
+                        if ((tid & 15) == 0) {
+                            p.scale_cache[row] = sc[0];
+                            p.scale_cache[(size_t)p.P * p.H * p.S + row] = sc[1];
+                        }
+                        store_key_word<CPL>(p.key_cache + row * (D / 2) + l * (CPL / 2), t[0]);
+                        uint32_t* words = (uint32_t*)(p.value_cache + (row - col) * (D / 2)) +
+                                          2 * l * CPL + (col >> 3);
+                        const uint32_t sh = 4u * (col & 7u);
+#pragma unroll
+                        for (int j = 0; j < CPL; ++j)
+                            words[2 * j] = (words[2 * j] & ~(0xfu << sh)) |
+                                           (((t[1][j] ^ 8u) & 0xfu) << sh);
+                    }
                 }
             }
         }
     }
 }
 
+// Which of the chunks c .. c + m - 1 (m <= kGroup) of a request (n tokens at
+// t0, the first at place a of its strip) share a strip with a token outside
+// them, into found[v ..]: their strips go into a table, and every slot of the
+// request is looked up in it, once for all of them. A chunk with several strips
+// stays out of the table (scatter_chunk finds it).
+__device__ __forceinline__ void scatter_search(const ScatterArgs& p, SearchShared& s, uint32_t t0,
+                                               uint32_t n, uint32_t a, uint32_t c, uint32_t v,
+                                               uint32_t m)
+{
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));  // nothing derived from it is held for long
+    const int row = tid >> 4, j16 = tid & 15;
+    const int64_t at = (int64_t)c * kStrip - a + tid;
+    const int32_t slot =
+        (uint32_t)row < m && at >= 0 && at < (int64_t)n ? p.slots[t0 + (uint32_t)at] : -1;
+    s.table[tid] = kNoStrip;
+    if (tid == 0) s.clash = 0;
+    lds_barrier();
+    const bool ok = slot_in_pool(slot, p.S, p.P);
+    const int sh = tid & 48;
+    const uint32_t vmask = (uint32_t)(__ballot(ok) >> sh) & 0xffffu;
+    const int32_t strip = __shfl(slot, sh + (vmask != 0 ? __builtin_ctz(vmask) : 0), 64) >> 4;
+    const bool several = ((uint32_t)(__ballot(ok && (slot >> 4) != strip) >> sh) & 0xffffu) != 0;
+    if (j16 == 0 && vmask != 0 && !several) {
+        for (uint32_t x = (uint32_t)strip % kTable;; x = (x + 1) % kTable) {
+            const int32_t was = atomicCAS(&s.table[x], kNoStrip, strip);
+            if (was == kNoStrip) s.owner[x] = (uint32_t)row;
+            if (was == strip) atomicOr(&s.clash, 1u << row);  // another chunk's as well
+            if (was == kNoStrip || was == strip) break;       // at most kGroup of kTable are taken
+        }
+    }
+    lds_barrier();
+    const int32_t* sl = p.slots + t0;
+    uint32_t hit = 0;
+    for (uint64_t ub = 0; ub < n; ub += 8 * kWriterThreads) {  // eight loads in flight a thread
+        int32_t st[8], e[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            st[k] = sl[min((uint32_t)ub + k * kWriterThreads + tid, n - 1)] >> 4;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) e[k] = s.table[(uint32_t)st[k] % kTable];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            uint32_t x = (uint32_t)st[k] % kTable;
+            while (e[k] != kNoStrip && e[k] != st[k]) {
+                x = (x + 1) % kTable;
+                e[k] = s.table[x];
+            }
+            if (e[k] == st[k]) {
+                const uint32_t u = min((uint32_t)ub + k * kWriterThreads + tid, n - 1);
+                if (((u + a) >> 4) != c + s.owner[x]) hit |= 1u << s.owner[x];
+            }
+        }
+    }
+    if (hit != 0) atomicOr(&s.clash, hit);
+    lds_barrier();
+    if ((uint32_t)tid < m) s.found[(v + tid) % kSearchRun] = (uint8_t)((s.clash >> tid) & 1u);
+    lds_barrier();
+}
+
 // One chunk of 16 tokens (first .. first + 15 of the request's n at t0), heads
-// [h0, h1). False: nothing is written, the chunk goes token by token.
+// [h0, h1). searched: no token outside the chunk touches its strip (known
+// already). False: nothing is written, the chunk goes token by token.
 template <int D>
 __device__ __forceinline__ bool scatter_chunk(const ScatterArgs& p, uint32_t t0, uint32_t n,
-                                              int64_t first, uint32_t h0, uint32_t h1,
-                                              const float (&sign)[D / 16],
+                                              int64_t first, bool searched, uint32_t h0,
+                                              uint32_t h1, const float (&sign)[D / 16],
                                               uint32_t (*lds_t)[D / 8][20], int* clash_w)
 {
     constexpr int CPL = D / 16;
@@ -549,7 +650,7 @@ __device__ __forceinline__ bool scatter_chunk(const ScatterArgs& p, uint32_t t0,
     const bool regular = __ballot(odd) == 0;
     // does another token of the request touch the strip?
     int clash = !regular;
-    if (regular) {
+    if (regular && !searched) {
         // eight loads in flight a thread (past the end: the last token again)
         const int32_t* sl = p.slots + t0;
         const uint32_t f = (uint32_t)first;  // mod 2^32, as the distance below
@@ -636,10 +737,23 @@ __device__ __forceinline__ bool scatter_chunk(const ScatterArgs& p, uint32_t t0,
     return true;
 }
 
+// The inclusive prefix sum over a wave: four shifts within the rows of 16
+// lanes, then each row's last lane added to the next rows.
+__device__ __forceinline__ uint32_t wave_prefix(uint32_t v)
+{
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);  // row_shr 1
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);  // row_shr 2
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);  // row_shr 4
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);  // row_shr 8
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);  // row_bcast 15
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);  // row_bcast 31
+    return v;
+}
+
 // The lengths are on the device only, so the grid is fixed: every workgroup
-// counts the requests' chunks (a prefix over the requests of the window,
-// staged in LDS; a request of n tokens has at most (n + 30) / 16 chunks) and
-// takes an equal run of the (chunk, head) pairs.
+// counts the requests' chunks (blocks of 64 requests to the waves in turn, a
+// prefix over each in LDS and one over the blocks) and takes an equal run of the
+// (chunk, head) pairs.
 template <int D>
 __global__ __launch_bounds__(kWriterThreads, D == 256 ? 3 : 4) void scatter_writer(
     ScatterArgs p, const float* __restrict__ pi_signs, const int32_t* __restrict__ cu_seqlens,
@@ -649,13 +763,15 @@ __global__ __launch_bounds__(kWriterThreads, D == 256 ? 3 : 4) void scatter_writ
     constexpr int CPL = D / 16;
     __shared__ __align__(16) uint32_t lds_t[2][D / 8][20];
     __shared__ __align__(16) int clash_w[kWriterThreads / 64];
-    // the requests: inclusive prefix of their chunks, first token, length, and
-    // the first token's place in its strip; read once here, so a chunk does not
-    // begin with two more dependent loads (the two cases above: 18.0 -> 17.5
-    // and 16.2 -> 15.5 us; 32 requests of 8 tokens 5.5 -> 5.2)
+    __shared__ SearchShared search;
+    // the requests: inclusive prefix of their chunks within their 64, first
+    // token, length, and the first token's place in its strip; read once here,
+    // so a chunk does not begin with two more dependent loads
     __shared__ uint32_t chunks[kScatterPlan], starts[kScatterPlan], counts[kScatterPlan];
     __shared__ uint8_t places[kScatterPlan];
+    __shared__ uint32_t sums[kScatterPlan / 64];
     const int tid = threadIdx.x, lane = tid & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
     if (probe != nullptr && blockIdx.x == 0 && tid < 32) {
         const int32_t fields[4] = {0, (int32_t)probe_grid, 1, (int32_t)item_count};
@@ -671,66 +787,77 @@ __global__ __launch_bounds__(kWriterThreads, D == 256 ? 3 : 4) void scatter_writ
     for (uint64_t rb = r0; rb < r1; rb += kScatterPlan) {
         const uint32_t nr = (uint32_t)min((uint64_t)kScatterPlan, r1 - rb);
         const int32_t* cu = cu_seqlens + rb;
-        if (tid < 64) {
-            uint32_t carry = 0;
-            for (uint32_t b = 0; b < nr; b += 64) {
-                const uint32_t i = min(b + lane, nr - 1);
-                const uint32_t t0 = (uint32_t)cu[i], t1 = (uint32_t)cu[i + 1];
-                const uint32_t n = t1 > t0 ? t1 - t0 : 0u;
-                const int32_t s0 = n > 0 ? p.slots[t0] : -1;
-                uint32_t v = b + lane < nr && n > 0 ? (n + 30u) >> 4 : 0u;
-#pragma unroll
-                for (int o = 1; o < 64; o <<= 1) {
-                    const uint32_t w = __shfl_up(v, o, 64);
-                    if (lane >= o) v += w;
-                }
-                v += carry;
-                if (b + lane < nr) {
-                    chunks[i] = v;
-                    starts[i] = t0;
-                    counts[i] = n;
-                    places[i] = s0 >= 0 ? s0 % kStrip : 0;
-                }
-                carry = __shfl(v, 63, 64);
-            }
+#pragma unroll 1
+        for (uint32_t b = wave; 64 * b < nr; b += kWriterThreads / 64) {
+            const uint32_t i = min(64 * b + lane, nr - 1);
+            const uint32_t t0 = (uint32_t)cu[i], t1 = (uint32_t)cu[i + 1];
+            const uint32_t n = 64 * b + lane < nr && t1 > t0 ? t1 - t0 : 0u;
+            const int32_t s0 = n > 0 ? p.slots[t0] : 0;
+            const uint32_t place = s0 >= 0 ? (uint32_t)s0 % kStrip : 0u;
+            const uint32_t v = wave_prefix(n > 0 ? (n + place + 15u) >> 4 : 0u);
+            if (lane == 63) sums[b] = v;
+            chunks[64 * b + lane] = v;
+            starts[64 * b + lane] = t0;
+            counts[64 * b + lane] = n;
+            places[64 * b + lane] = (uint8_t)place;
         }
         lds_barrier();
+        // lane b: the chunks up to and with block b of 64 requests
+        const uint32_t blocks = wave_prefix(64u * lane < nr ? sums[lane] : 0u);
+        auto before = [&](uint32_t b) -> uint32_t {
+            return b > 0 ? __builtin_amdgcn_readlane(blocks, b - 1) : 0u;
+        };
+        // the prefix up to and with request i
+        auto upto = [&](uint32_t i) -> uint32_t {
+            return __builtin_amdgcn_readfirstlane(chunks[i]) + before(i / 64);
+        };
         // an equal run of (chunk, head) pairs to every workgroup
-        const uint32_t total = __builtin_amdgcn_readfirstlane(chunks[nr - 1]);
+        const uint32_t total = __builtin_amdgcn_readlane(blocks, 63);
         const uint64_t pairs = (uint64_t)total * p.H;
         const uint64_t per = (pairs + kScatterGrid<D> - 1) / kScatterGrid<D>;
         const uint64_t at = per * blockIdx.x;
         uint32_t v = pairs <= 0xffffffffull ? (uint32_t)at / p.H : (uint32_t)(at / p.H);
         uint32_t h = (uint32_t)(at - (uint64_t)v * p.H);
-        uint32_t i = nr;  // the first request whose prefix passes v
-        for (uint32_t b = 0; b < nr && at < pairs; b += 64) {
-            const uint64_t m = __ballot(b + lane < nr && chunks[b + lane] > v);
-            if (m != 0) {
-                i = b + (uint32_t)__builtin_ctzll(m);
-                break;
-            }
+        uint32_t i = 0;  // the first request whose prefix passes v
+        if (at < pairs) {
+            const uint32_t b = (uint32_t)__builtin_ctzll(__ballot(blocks > v));
+            i = 64 * b + (uint32_t)__builtin_ctzll(__ballot(chunks[64 * b + lane] + before(b) > v));
         }
-        i = __builtin_amdgcn_readfirstlane(i);
-        for (uint64_t left = per; left > 0 && i < nr;) {
-            const uint32_t take = (uint32_t)min(left, (uint64_t)(p.H - h));
-            const uint32_t c =
-                v - (i > 0 ? __builtin_amdgcn_readfirstlane(chunks[i - 1]) : 0u);
+        // (a workgroup's run is far below 2^32: its rows are in memory)
+        uint32_t left = at < pairs ? (uint32_t)min(per, pairs - at) : 0u;
+        uint32_t known = 0;  // the run's chunks before this one are searched
+        if (__builtin_expect(left > p.H - h &&
+                                 __builtin_amdgcn_readfirstlane(counts[i]) > kSearchFrom,
+                             0)) {
+            const uint32_t begin = i > 0 ? upto(i - 1) : 0u;
+            known = min(min(upto(i), v + kSearchRun), v + (left + h + p.H - 1) / p.H);
+            for (uint32_t x = v; x < known; x += kGroup)
+                scatter_search(p, search, __builtin_amdgcn_readfirstlane(starts[i]),
+                               __builtin_amdgcn_readfirstlane(counts[i]),
+                               __builtin_amdgcn_readfirstlane((uint32_t)places[i]), x - begin, x,
+                               min(kGroup, known - x));
+        }
+        while (left > 0) {
+            const uint32_t take = min(left, p.H - h);
+            const uint32_t c = v - (i > 0 ? upto(i - 1) : 0u);
             const uint64_t item0 = (rb + i) * p.H;  // the request's heads inside the window
             const uint32_t h0 = (uint32_t)(max(item0 + h, (uint64_t)item_begin) - item0);
             const uint32_t h1 = (uint32_t)(min(item0 + h + take, item_end) - item0);
             const uint32_t t0 = __builtin_amdgcn_readfirstlane(starts[i]);
             const uint32_t n = __builtin_amdgcn_readfirstlane(counts[i]);
-            const int64_t first =
-                (int64_t)c * kStrip - __builtin_amdgcn_readfirstlane((int)places[i]);
-            if ((int32_t)(h1 - h0) > 0 && first < (int64_t)n) {
-                if (!scatter_chunk<D>(p, t0, n, first, h0, h1, sign, lds_t, clash_w))
+            const uint32_t place = __builtin_amdgcn_readfirstlane((uint32_t)places[i]);
+            const int64_t first = (int64_t)c * kStrip - place;
+            if ((int32_t)(h1 - h0) > 0) {
+                if ((v < known && __builtin_amdgcn_readfirstlane(search.found[v % kSearchRun])) ||
+                    !scatter_chunk<D>(p, t0, n, first, v < known || n + place <= kStrip, h0, h1,
+                                      sign, lds_t, clash_w))
                     scatter_tokens<D>(p, t0, n, first, h0, h1, sign);
             }
             lds_barrier();  // the next chunk writes clash_w and the first buffer again
             left -= take;
             h = 0;
             ++v;
-            while (i < nr && __builtin_amdgcn_readfirstlane(chunks[i]) <= v) ++i;
+            while (left > 0 && upto(i) <= v) ++i;
         }
         lds_barrier();
     }

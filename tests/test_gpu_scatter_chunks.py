@@ -105,3 +105,45 @@ def test_extreme_rows(tq4, oracle, d):
     scale = np.exp2(rng.integers(-132, 120, (sum(lens), 1, 1)).astype(np.float64))
     scale[::7] = 0.0
     case(tq4, oracle, rng, lens, ["prompt"] * 3, 2, d, 16, scale=scale)
+
+
+@pytest.mark.parametrize("R", [1, 3, 1023, 1024, 1025, 2050])
+@pytest.mark.parametrize("H", [1, 3])
+def test_request_counts_around_the_staged_plan(tq4, oracle, R, H):
+    """Request counts at the edges of the on-chip plan (1024 requests, four a
+    thread), empty ones and short and longer ones among them."""
+    rng = np.random.default_rng(80 + R + H)
+    lens = [int(x) for x in rng.choice([0, 1, 1, 2, 5, 16, 17, 40], R)]
+    lens[-1] = 19
+    case(tq4, oracle, rng, lens, ["prompt"] * R, H, 64, 16)
+
+
+@pytest.mark.parametrize("kind,n", [("prompt", 270001), ("rewritten", 40000), ("pads", 40000)])
+def test_more_chunks_than_a_group(tq4, oracle, kind, n):
+    """Requests of more chunks than the workgroups check together (16 each, 1024
+    workgroups), regular and with strips that far chunks share."""
+    case(tq4, oracle, np.random.default_rng(n), [n, 7], [kind, "prompt"], 1, 64, 16)
+
+
+@pytest.mark.parametrize("tail", ["plain", "shared", "swapped"])
+def test_strips_of_one_table_place(tq4, oracle, tail):
+    """The strips of a group's chunks all at one place of the strip table (equal
+    modulo 256), a chunk that touches another's strip again, two chunks with
+    their strips' halves swapped."""
+    rng = np.random.default_rng(81)
+    H, d, S, chunks = 2, 64, 16, 40
+    P = 256 * chunks
+    strips = 256 * rng.permutation(chunks) + 5
+    slots = (strips[:, None] * 16 + np.arange(16)).reshape(-1)
+    if tail == "shared":
+        slots[-16:] = slots[48:64]
+    elif tail == "swapped":
+        slots[32:40], slots[320:328] = slots[320:328].copy(), slots[32:40].copy()
+    T = len(slots)
+    key, val = (f32_to_bf16(rng.standard_normal((T, H, d)).astype(np.float32)) for _ in range(2))
+    nb = P * H * S * d // 2
+    prior = (rng.integers(-128, 128, nb, dtype=np.int8), rng.integers(-128, 128, nb, dtype=np.int8),
+             rng.standard_normal(2 * P * H * S).astype(np.float32))
+    got, want = scatter_pair(tq4, oracle, key, val, slots.astype(np.int32),
+                             np.array([0, T], np.int32), 1, H, d, S, P, prior=prior)
+    assert_same(got, want)
