@@ -16,6 +16,7 @@
 #include <Python.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 #include <cmath>
 #include <cstring>
@@ -640,4 +641,10 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_tq4_host",
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__tq4_host(void) { return PyModule_Create(&kModule); }
+PyMODINIT_FUNC PyInit__tq4_host(void)
+{
+    PyObject* m = PyModule_Create(&kModule);
+    // the torch whose headers this was built with: tq4.py binds no other
+    if (m && PyModule_AddStringConstant(m, "torch_version", TORCH_VERSION) != 0) Py_CLEAR(m);
+    return m;
+}

@@ -25,6 +25,8 @@ from __future__ import annotations
 import ctypes as C
 import math
 import os
+import sysconfig
+import warnings
 
 import torch  # noqa: F401  (loads torch's HIP runtime first; libtq4 binds to it)
 
@@ -129,16 +131,26 @@ def lib():
 
 
 def _bind_host(L):
+    """Binds the native checks where they are built and fit this Python and torch;
+    otherwise (with a warning where a build of them is there) the Python ones
+    take every call."""
     global _fast
-    if not os.path.exists(os.path.join(_HERE, "_tq4_host.so")):
+    if not os.path.exists(os.path.join(_HERE, "_tq4_host" + sysconfig.get_config_var("EXT_SUFFIX"))):
         return
-    from . import _tq4_host as host
-    host.bind({n: C.cast(getattr(L, n), _P).value for n in (
-        "tq4_reshape_and_cache_a8", "tq4_reshape_and_cache_bf16", "tq4_reshape_scatter",
-        "tq4_decode_auto_splits", "tq4_paged_decode", "tq4_paged_decode_partials",
-        "tq4_splitk_combine", "tq4_rms_reshape_and_cache", "tq4_icdf_quantize",
-        "tq4_lloydmax_quantize", "tq4_kv4fp8_workspace_bytes", "tq4_kv4fp8_decode",
-        "tq4_kv4fp8_decode_raw_query")})
+    try:
+        from . import _tq4_host as host
+        if host.torch_version != torch.__version__.split("+")[0]:
+            raise ImportError(f"built for torch {host.torch_version}, this is {torch.__version__}")
+        host.bind({n: C.cast(getattr(L, n), _P).value for n in (
+            "tq4_reshape_and_cache_a8", "tq4_reshape_and_cache_bf16", "tq4_reshape_scatter",
+            "tq4_decode_auto_splits", "tq4_paged_decode", "tq4_paged_decode_partials",
+            "tq4_splitk_combine", "tq4_rms_reshape_and_cache", "tq4_icdf_quantize",
+            "tq4_lloydmax_quantize", "tq4_kv4fp8_workspace_bytes", "tq4_kv4fp8_decode",
+            "tq4_kv4fp8_decode_raw_query")})
+    except ImportError as e:
+        warnings.warn(f"_tq4_host is not used: {e}; build it again (make -C csrc host) or remove it",
+                      RuntimeWarning, stacklevel=3)
+        return
     _fast = host
 
 
