@@ -166,14 +166,22 @@ bool shape3(const at::Tensor* t, Shape3& s)
     return small(s.a) && small(s.b) && small(s.c) && t->numel() > 0;
 }
 
+// a * b, at most 2^63 - 1: more elements than any tensor holds, as Python's
+// unbounded product would be.
+uint64_t mul(uint64_t a, uint64_t b)
+{
+    uint64_t r;
+    return __builtin_mul_overflow(a, b, &r) || r > (uint64_t)INT64_MAX ? (uint64_t)INT64_MAX : r;
+}
+bool at_least(const at::Tensor* t, uint64_t n) { return t && (uint64_t)t->numel() >= n; }
+
 // The TQ4 cache of num_blocks pages (tq4.py _check_cache).
 bool cache_ok(const at::Tensor* kc, const at::Tensor* vc, const at::Tensor* sc, uint64_t blocks,
               uint64_t heads, uint64_t block_size, uint64_t d)
 {
-    const uint64_t rows = blocks * heads * block_size;
-    return blocks * heads < (1ull << 40) && kc && vc && sc &&
-           (uint64_t)kc->numel() >= rows * d / 2 && (uint64_t)vc->numel() >= rows * d / 2 &&
-           (uint64_t)sc->numel() >= 2 * rows;
+    const uint64_t rows = mul(mul(blocks, heads), block_size);
+    return at_least(kc, mul(rows, d) / 2) && at_least(vc, mul(rows, d) / 2) &&
+           at_least(sc, mul(rows, 2));
 }
 
 // The pages of a pool given by its key cache alone (num_blocks None); -1 when
@@ -181,8 +189,8 @@ bool cache_ok(const at::Tensor* kc, const at::Tensor* vc, const at::Tensor* sc, 
 int64_t pool_pages(const at::Tensor* kc, const Shape3& s, uint32_t S)
 {
     if (!kc || S == 0) return -1;
-    const int64_t pages = kc->numel() * 2 / (s.b * (int64_t)S * s.c);
-    return small(pages) ? pages : -1;
+    const uint64_t pages = mul(kc->numel(), 2) / mul(mul(s.b, S), s.c);
+    return small((int64_t)pages) ? (int64_t)pages : -1;
 }
 
 bool holds(const at::Tensor* t, int64_t n) { return !t || t->numel() >= n; }
@@ -334,9 +342,9 @@ PyObject* paged_decode_partials(PyObject*, PyObject* const* a, Py_ssize_t n)
         const float scale = g.real(inv_sqrt(d.s.c)), isl = g.real(inv_sqrt(d.s.c));
         const uint32_t flags = g.num();
         void* st = g.stream();
-        const int64_t need = d.s.a * d.s.b * (int64_t)K * (d.s.c + 4);
-        if (!g.need(K > 0 && K <= TQ4_MAX_SPLITS && (ws_obj == Py_None || ws) &&
-                    holds(ws, need) && (d.pi || (flags & TQ4_DECODE_QUERY_ROTATED))))
+        const uint64_t need = mul(mul(mul(d.s.a, d.s.b), K), d.s.c + 4);
+        if (!g.need(K > 0 && K <= TQ4_MAX_SPLITS && (ws_obj == Py_None || at_least(ws, need)) &&
+                    (d.pi || (flags & TQ4_DECODE_QUERY_ROTATED))))
             return nullptr;
         at::Tensor fresh;
         if (!ws) {
@@ -375,7 +383,7 @@ PyObject* splitk_combine(PyObject*, PyObject* const* a, Py_ssize_t n)
         void* st = g.stream();
         const uint64_t rows = (uint64_t)B * Hq;
         if (!g.need(rows > 0 && rows < (1ull << 31) && d <= 256 && K > 0 && K <= TQ4_MAX_SPLITS &&
-                    (uint64_t)ws->numel() >= rows * K * (d + 4) && (pi || stage == 0) &&
+                    at_least(ws, mul(rows * K, d + 4)) && (pi || stage == 0) &&
                     holds(pi, d) && (!gate || (uint64_t)gate->numel() == rows * d) &&
                     (out_obj == Py_None || (out && (uint64_t)out->numel() == rows * d))))
             return nullptr;
@@ -413,10 +421,9 @@ PyObject* rms_reshape_and_cache(PyObject*, PyObject* const* a, Py_ssize_t n)
         const float isl = g.real(inv_sqrt(s.c));
         const uint32_t grid = g.num(), tpc = g.num();
         void* st = g.stream();
-        const uint64_t slots = (uint64_t)P * S, row = (uint64_t)s.b * s.c / 2;
-        if (!g.need(slots > 0 && slots < (1ull << 40) && (uint64_t)kc->numel() >= slots * row &&
-                    (uint64_t)vc->numel() >= slots * row &&
-                    (uint64_t)sc->numel() >= slots * ((2 * (uint64_t)s.b + 7) / 8 * 8) &&
+        const uint64_t slots = (uint64_t)P * S, half = mul(mul(slots, s.b), s.c) / 2;
+        if (!g.need(slots > 0 && at_least(kc, half) && at_least(vc, half) &&
+                    at_least(sc, mul(slots, (2 * (uint64_t)s.b + 7) / 8 * 8)) &&
                     holds(sl, s.a) && holds(pi, s.c)))
             return nullptr;
         return PyLong_FromLong(unlocked([&] {
@@ -440,8 +447,8 @@ bool kv4_launch(tq4_kv4fp8_launch& L, uint64_t tokens, uint64_t heads, uint64_t 
         return false;
     const uint64_t group = heads / kv_heads;
     const uint64_t chunk = heads_per_task < group ? heads_per_task : group;
-    const uint64_t tasks = tokens * kv_heads * splits * ((group + chunk - 1) / chunk);
-    if (tasks == 0 || tasks > 0x7fffffffull || tokens * heads > 0x7fffffffull) return false;
+    const uint64_t tasks = mul(mul(mul(tokens, kv_heads), splits), (group + chunk - 1) / chunk);
+    if (tasks == 0 || tasks > 0x7fffffffull || mul(tokens, heads) > 0x7fffffffull) return false;
     const uint64_t tpb = (tasks + 31) / 32, grid = (tasks + tpb - 1) / tpb;
     std::memset(&L, 0, sizeof L);
     L.grid = (uint32_t)grid;
@@ -495,9 +502,8 @@ PyObject* kv4fp8_decode(PyObject*, PyObject* const* a, Py_ssize_t n)
         if (!g.need(shape3(q, s) && s.c == 256 && H > 0 && S > 0 && P > 0)) return nullptr;
         const uint64_t rows = (uint64_t)P * S;
         const int64_t numel = q->numel();
-        if (!g.need(rows < (1ull << 40) && (uint64_t)kc->numel() >= rows * H * 128 &&
-                    (uint64_t)vc->numel() >= rows * H * 128 &&
-                    (uint64_t)sc->numel() >= rows * 8 && bt->dim() == 2 && bt->size(0) == s.a &&
+        if (!g.need(at_least(kc, mul(mul(rows, H), 128)) && at_least(vc, mul(mul(rows, H), 128)) &&
+                    at_least(sc, mul(rows, 8)) && bt && cl && bt->dim() == 2 && bt->size(0) == s.a &&
                     cl->numel() == s.a && (!raw || (pi && pi->numel() >= 256)) &&
                     (!gate || gate->numel() == numel) && (!q_out || q_out->numel() == numel) &&
                     (out_obj == Py_None || (out && out->numel() == numel))))

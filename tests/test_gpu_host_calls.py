@@ -137,6 +137,32 @@ def test_refused_call_same_message(tq4, name):
     assert refused or name.startswith(("icdf", "lloyd"))
 
 
+@pytest.mark.parametrize("name", NAMES)
+def test_refused_number_same_message(tq4, name):
+    """Each size argument, and the pool's page count and page size together, at
+    zero and so large that the pool's size passes 2^64: where Python refuses the
+    call, the native route ends in the same refusal."""
+    import inspect
+    tq4.lib()
+    args, kwargs = _calls()[name]
+    bound = inspect.signature(getattr(tq4, name.split(":")[0])).bind(*args, **kwargs)
+    bound.apply_defaults()
+    call = dict(bound.arguments)
+    numbers = [k for k in ("num_blocks", "block_size", "num_kv_heads", "kv_heads", "num_requests",
+                           "num_seqs", "num_heads", "head_size") if k in call]
+    big = (1 << 30, (1 << 31) - 1, 1 << 31, 1 << 40)
+    tries = [{k: v} for k in numbers for v in (0, *big)]
+    if "num_blocks" in call:
+        tries += [dict(num_blocks=a, block_size=b) for a in (1, *big) for b in big]
+    refused = 0
+    for over in tries:
+        want = _run(tq4, name, (), {**call, **over}, native=False)
+        if isinstance(want, tuple):
+            refused += 1
+            assert _run(tq4, name, (), {**call, **over}, native=True) == want, over
+    assert refused or not numbers
+
+
 def test_other_streams_and_threads(tq4):
     """The call goes to torch's current stream of its thread, or the one given."""
     import threading
