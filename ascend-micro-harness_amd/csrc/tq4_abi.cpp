@@ -322,7 +322,8 @@ int decode_checks(const uint16_t* q, const int8_t* kc, const int8_t* vc, const f
         return TQ4_ERR_FLAGS;
     if (!(flags & TQ4_DECODE_QUERY_ROTATED) && !pi_signs) return TQ4_ERR_ROTATION;
     // cache rows are indexed in 32 bits on the device
-    if ((uint64_t)num_blocks * num_kv_heads * block_size > 0xffffffffull) return TQ4_ERR_RANGE;
+    // (divided: the product of the three passes 64 bits)
+    if ((uint64_t)num_blocks * num_kv_heads > 0xffffffffull / block_size) return TQ4_ERR_RANGE;
     return TQ4_OK;
 }
 

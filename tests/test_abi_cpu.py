@@ -356,3 +356,13 @@ def test_auto_splits_skewed_lengths(lib):
     assert power(60, 8, 1744, 1) == 1 and power(42, 8, 900, 6) == 1
     assert power(106, 2, 13818, 1.5) == 3 and power(106, 2, 13818, 4) == 4
     assert power(32, 8, 12129, 1.3) == 4 and power(128, 2, 16117, 0.55) == 2
+
+
+def test_decode_row_count_past_64_bits(lib):
+    """num_blocks * num_kv_heads * block_size is refused past 2^32 - 1 rows also
+    where the product passes 2^64 (2^31 * 4 * 2^31 is 0 in 64 bits)."""
+    fake = C.c_void_p(4096)  # never dereferenced: refused before any HIP call
+    for heads, pages, page in ((4, 1 << 31, 1 << 31), (4, 1 << 30, 1 << 30), (1, 1 << 20, 4096)):
+        rc = lib.tq4_paged_decode(None, *[fake] * 7, None, fake, C.c_size_t(1 << 30), fake, 1, 4, heads,
+                                  128, page, pages, 1, 1, C.c_float(1.0), C.c_float(1.0), 0, 0)
+        assert rc == -10, (heads, pages, page, rc)
