@@ -150,24 +150,21 @@ __global__ __launch_bounds__(kRmsThreads) void rms_writer(
     for (int j = 0; j < CPL; ++j) sg[j] = pi_signs[l * CPL + j];
     if (slot < 0 || (uint64_t)slot >= slot_count) return;  // a pad token or a slot past the pool
 
-    // ApplyPi: signs, FWHT at strides 1 .. D/2, x inv_sqrt_len, signs. The
-    // first signs flip the 16-bit values' sign bits, two at a time. The FWHT's
-    // cross-lane stages run on sign-tracked values (row_fmac_stage): v holds
-    // sigma * y afterwards, sigma = row_sigma(l)
+    // ApplyPi: signs, FWHT at strides 1 .. D/2, x inv_sqrt_len, signs (products:
+    // any float is taken). The FWHT's cross-lane stages run on sign-tracked
+    // values (row_fmac_stage): v holds sigma * y afterwards, sigma = row_sigma(l)
     float v[2][CPL];
 #pragma unroll
     for (int j = 0; j < CPL; j += 2) {
-        const uint32_t flip = (__float_as_uint(sg[j]) & 0x80000000u) >> 16 |
-                              (__float_as_uint(sg[j + 1]) & 0x80000000u);
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
-            const uint32_t w = raw[r][j / 2] ^ flip;
+            const uint32_t w = raw[r][j / 2];
             if constexpr (IN_BF16) {
-                v[r][j] = __uint_as_float(w << 16);
-                v[r][j + 1] = __uint_as_float(w & 0xffff0000u);
+                v[r][j] = __uint_as_float(w << 16) * sg[j];
+                v[r][j + 1] = __uint_as_float(w & 0xffff0000u) * sg[j + 1];
             } else {
-                v[r][j] = (float)__builtin_bit_cast(_Float16, (uint16_t)w);
-                v[r][j + 1] = (float)__builtin_bit_cast(_Float16, (uint16_t)(w >> 16));
+                v[r][j] = (float)__builtin_bit_cast(_Float16, (uint16_t)w) * sg[j];
+                v[r][j + 1] = (float)__builtin_bit_cast(_Float16, (uint16_t)(w >> 16)) * sg[j + 1];
             }
         }
     }
@@ -190,14 +187,10 @@ __global__ __launch_bounds__(kRmsThreads) void rms_writer(
             }
         }
     }
-    // x inv_sqrt_len, then the sign: one product with the signed factor (the
-    // sign is +-1, so the rounding is the same)
-#pragma unroll
-    for (int j = 0; j < CPL; ++j) sg[j] = inv_sqrt_len * sg[j];
 #pragma unroll
     for (int r = 0; r < 2; ++r) {
 #pragma unroll
-        for (int j = 0; j < CPL; ++j) v[r][j] = v[r][j] * sg[j];
+        for (int j = 0; j < CPL; ++j) v[r][j] = (v[r][j] * inv_sqrt_len) * sg[j];
     }
 
     // scale = sqrt(sum y^2) * inv_sqrt_len + eps: per-lane sequential sum, then

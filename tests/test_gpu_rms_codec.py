@@ -25,7 +25,7 @@ def to_elem(x, bf16):
     return x.astype(np.float16).view(np.uint16)
 
 
-def run_case(tq4, oracle, T, H, d, S, P, bf16, seed, block_dim=0, tpc=0):
+def run_case(tq4, oracle, T, H, d, S, P, bf16, seed, block_dim=0, tpc=0, signs=None):
     rng = np.random.default_rng(seed)
     mags = rng.choice([1e-18, 1e-3, 1.0, 30.0, 1e4 if bf16 else 100.0], size=(T, H, 1))
     key = to_elem(rng.standard_normal((T, H, d)) * mags, bf16)
@@ -40,7 +40,8 @@ def run_case(tq4, oracle, T, H, d, S, P, bf16, seed, block_dim=0, tpc=0):
     kc, vc, sc = canary_bytes(nb), canary_bytes(nb), canary_floats(P * S * ssf)
     o = [kc.copy(), vc.copy(), sc.copy()]
     isl = np.float32(1 / math.sqrt(d))
-    signs = np.where(rng.random(d) < 0.5, -1.0, 1.0).astype(np.float32)
+    if signs is None:
+        signs = np.where(rng.random(d) < 0.5, -1.0, 1.0).astype(np.float32)
     limit = min(T, block_dim * tpc) if block_dim else T
     oracle.rms_reshape_and_cache(1 if bf16 else 0, key, val, o[0], o[1], o[2], slots, signs, H,
                                  d, S, P, limit, isl)
@@ -164,3 +165,13 @@ def test_writer_item_and_scale_record_edges(tq4, oracle, T, H, d):
     """Item counts around a workgroup's sixteen, head counts that the index
     multiplier and the scale record's zero padding treat differently."""
     run_case(tq4, oracle, max(T, 2), H, d, 16, 4, bool(T % 2), seed=T * 100 + H + d)
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("bf16", [True, False])
+def test_writer_sign_values(tq4, oracle, d, bf16):
+    """Pi = diag(s) H diag(s) for any s: both factors are products, whatever the
+    magnitude (the rounding of each included)."""
+    rng = np.random.default_rng(d + bf16)
+    s = rng.choice([1.0, -1.0, 0.5, -2.0, 0.0, -0.0, 1.1, -0.3], d).astype(np.float32)
+    run_case(tq4, oracle, 50, 3, d, 16, 8, bf16, seed=d, signs=s)
