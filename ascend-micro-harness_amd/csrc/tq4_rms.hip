@@ -96,14 +96,15 @@ static_assert(kPos[0] * 4 != 1 && kPos[1] * 4 != 2 && kPos[2] * 4 != 3 && kPos[3
               "no threshold but 0 on a bin boundary");
 
 // The codec's level of z = y * (1/scale): #{i : t_i < z} (NaN -> 0). lut:
-// kBins staged in LDS. The bin is the truncated 4z + 11 (a negative sum and a
-// NaN give 0); where that sum's rounding crosses a bin's end, no threshold
+// kBins staged in LDS. The bin is the truncated 4z + 11, held within the table
+// before the conversion (v_med3 of a NaN is the smaller bound); where that sum's rounding crosses a bin's end, no threshold
 // lies between z and the end, so both bins give the same count.
 __device__ __forceinline__ uint32_t level_of(float z, const LevelBin* lut)
 {
     // 8 bytes an entry: the byte offset is the truncated 32z + 88, its low
     // bits dropped
-    const uint32_t u = min(__float2uint_rz(__builtin_fmaf(z, 32.0f, 88.0f)), 8u * kLevelBins - 1u);
+    const uint32_t u = (uint32_t)__builtin_amdgcn_fmed3f(__builtin_fmaf(z, 32.0f, 88.0f), 0.0f,
+                                                         (float)(8 * kLevelBins - 1));
     const LevelBin e = *(const LevelBin*)((const char*)lut + (u & ~7u));
     return e.below + (e.inside < z ? 1u : 0u);
 }

@@ -175,3 +175,34 @@ def test_writer_sign_values(tq4, oracle, d, bf16):
     rng = np.random.default_rng(d + bf16)
     s = rng.choice([1.0, -1.0, 0.5, -2.0, 0.0, -0.0, 1.1, -0.3], d).astype(np.float32)
     run_case(tq4, oracle, 50, 3, d, 16, 8, bf16, seed=d, signs=s)
+
+
+@pytest.mark.parametrize("bf16", [True, False])
+def test_writer_levels_beyond_the_bins(tq4, oracle, bf16):
+    """Values far outside the level bins on both sides (one channel of a row
+    carries nearly all of it), infinities and NaNs: the outermost levels, and
+    level 0 for a NaN."""
+    rng = np.random.default_rng(91 + bf16)
+    T, H, d, S, P = 40, 2, 128, 16, 4
+    x = rng.standard_normal((2, T, H, d)) * 1e-3
+    y = np.zeros((d,))
+    y[5] = 200.0
+    spike = hadamard(d) @ y / math.sqrt(d)  # Pi gives it back as one large value
+    x[:, ::3] = spike * rng.choice([-1.0, 1.0], (2, len(x[0, ::3]), H, 1))
+    x[0, 1, :, 7], x[0, 2, :, 7], x[1, 4, :, 9] = np.inf, -np.inf, np.nan
+    key, val = to_elem(x[0], bf16), to_elem(x[1], bf16)
+    slots, signs = rng.permutation(P * S)[:T].astype(np.int32), np.ones(d, np.float32)
+    isl = np.float32(1 / math.sqrt(d))
+    nb, ssf = P * S * H * d // 2, tq4.rms_scale_slot_floats(H)
+    kc, vc, sc = canary_bytes(nb), canary_bytes(nb), canary_floats(P * S * ssf)
+    o = [kc.copy(), vc.copy(), sc.copy()]
+    oracle.rms_reshape_and_cache(1 if bf16 else 0, key, val, *o, slots, signs, H, d, S, P, T, isl)
+    dt = torch.bfloat16 if bf16 else torch.float16
+    kt, vt = (torch.from_numpy(a.view(np.int16)).cuda().view(dt) for a in (key, val))
+    g = [dev(kc), dev(vc), dev(sc)]
+    tq4.rms_reshape_and_cache(kt, vt, *g, dev(slots), dev(signs), num_blocks=P, block_size=S,
+                              inv_sqrt_len=float(isl))
+    assert np.array_equal(host(g[0]), o[0]) and np.array_equal(host(g[1]), o[1])
+    got, want = host(g[2]), o[2]
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[~np.isnan(got)], want[~np.isnan(want)])
