@@ -30,9 +30,10 @@ def run_case(tq4, oracle, T, H, d, S, P, bf16, seed, block_dim=0, tpc=0, signs=N
     mags = rng.choice([1e-18, 1e-3, 1.0, 30.0, 1e4 if bf16 else 100.0], size=(T, H, 1))
     key = to_elem(rng.standard_normal((T, H, d)) * mags, bf16)
     val = to_elem(rng.standard_normal((T, H, d)) * mags[::-1], bf16)
-    key[0] = 0  # an all-zero token: scale 1e-20, every level 7
     slots = rng.permutation(P * S)[:T].astype(np.int32)
-    slots[1] = -1
+    if T > 1:
+        key[0] = 0  # an all-zero token: scale 1e-20, every level 7
+        slots[1] = -1
     if T > 3:
         slots[3] = P * S + 5  # past the pool
     ssf = tq4.rms_scale_slot_floats(H)
@@ -160,11 +161,11 @@ def hadamard(n):
 
 
 @pytest.mark.parametrize("d", [64, 128, 256])
-@pytest.mark.parametrize("T,H", [(2, 1), (17, 1), (33, 5), (5, 16), (7, 31), (1, 4)])
+@pytest.mark.parametrize("T,H", [(2, 1), (17, 1), (33, 5), (5, 16), (7, 31), (1, 4), (1, 1)])
 def test_writer_item_and_scale_record_edges(tq4, oracle, T, H, d):
     """Item counts around a workgroup's sixteen, head counts that the index
     multiplier and the scale record's zero padding treat differently."""
-    run_case(tq4, oracle, max(T, 2), H, d, 16, 4, bool(T % 2), seed=T * 100 + H + d)
+    run_case(tq4, oracle, T, H, d, 16, 4, bool(T % 2), seed=T * 100 + H + d)
 
 
 @pytest.mark.parametrize("d", [64, 128, 256])
