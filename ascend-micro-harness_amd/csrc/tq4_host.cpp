@@ -141,7 +141,8 @@ int unlocked(F&& f)
 }
 
 // f(Args) -> new reference, or nullptr for "take it in Python"; a C++
-// exception before the launch is the same.
+// exception before the launch is the same, unless Python code raised it (a
+// dispatch mode in an allocation): that one goes to the caller.
 template <class F>
 PyObject* entry(PyObject* const* a, Py_ssize_t n, F&& f)
 {
@@ -152,6 +153,7 @@ PyObject* entry(PyObject* const* a, Py_ssize_t n, F&& f)
             if (PyErr_Occurred()) return nullptr;
         }
     } catch (...) {
+        if (PyErr_Occurred()) return nullptr;
     }
     Py_RETURN_NONE;
 }

@@ -188,3 +188,24 @@ def test_other_streams_and_threads(tq4):
     torch.cuda.synchronize()
     assert len(got) == 6 and all(torch.equal(g, want) for g in got)
     assert math.isfinite(float(want.float().sum()))
+
+
+@pytest.mark.parametrize("name", ["paged_decode", "paged_decode_partials", "splitk_combine",
+                                  "kv4fp8_decode", "icdf_quantize", "lloydmax_quantize"])
+def test_exception_of_an_allocation(tq4, name):
+    """An exception that Python code raises out of the output's allocation (here a
+    dispatch mode) reaches the caller as it is."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+    tq4.lib()
+
+    class Refuse(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            if "empty" in str(func):
+                raise KeyError("no allocation here")
+            return func(*args, **(kwargs or {}))
+
+    args, kwargs = _calls()[name]
+    torch.cuda.synchronize()
+    with Refuse():
+        got = [_run(tq4, name, args, kwargs, native) for native in (False, True)]
+    assert got[0] == got[1] == ("KeyError", repr("no allocation here"))
