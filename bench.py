@@ -576,6 +576,37 @@ class Batch:
 
 
 # ---------------------------------------------------------------- main
+def line(result):
+    """The printed form of a result: the headline whole, every other row without
+    what its own figures or the headline's say already, so that the line stays
+    under 9,000 characters (readers of a log's end keep about 10,000)."""
+    def row(r, sweep):
+        if isinstance(r, list):
+            return [row(x, sweep) for x in r]
+        if not isinstance(r, dict):
+            return r
+        out = {}
+        for k, v in r.items():
+            if k == "roofline":
+                out.update({x: v[x] for x in ("frac", "traffic_ratio") if x in v})
+            elif k == "cpu_baseline":
+                out["cpu"] = None if v is None else [
+                    v["value"], v["unit"], v["cores"], (v.get("single_thread") or {}).get("value")]
+            elif k == "spread_us":
+                out["p99_us"] = v["p99_us"]
+            elif k in ("launches_per_sample", "samples", "pct_hbm_peak", "overhead_bytes") or (
+                    k in ("steps", "warmup", "algorithmic_bytes") and sweep) or (
+                    k == "poll_timeouts" and not v):
+                continue
+            else:
+                out[k] = row(v, sweep or k == "rows")
+        return out
+
+    head = ("config", "decode_us", "roofline", "cpu_baseline")
+    return {k: v if k in head or not isinstance(v, dict) else row(v, k == "split_sweep")
+            for k, v in result.items()}
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -585,6 +616,8 @@ def main():
                     help="CPU-leg budget of the headline row (other rows use less)")
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--no-extra", action="store_true", help="headline decode only")
+    ap.add_argument("--full", metavar="FILE",
+                    help="also write every row's whole record (spreads, rooflines, CPU legs)")
     ap.add_argument("--pmc-run", metavar="ROW",
                     help="one bench row's workload (8 or more launches of its kernel) plus a "
                          "plain copy of known size, for rocprofv3 --pmc; --pmc-rows lists them")
@@ -721,7 +754,10 @@ def main():
     if timeouts:
         result["INVALID"] = f"{timeouts} combine rows gave up their bounded poll"
     result.update(extra)
-    print(json.dumps(result), flush=True)
+    if args.full:
+        with open(args.full, "w") as f:
+            json.dump(result, f, indent=1)
+    print(json.dumps(line(result)), flush=True)
 
 
 PHASES = ["start", "phase-0 loads retired", "first strip pairs issued", "q operands built",

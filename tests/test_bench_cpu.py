@@ -142,3 +142,34 @@ def test_decode_overhead_bytes_closed_form():
     # a sequence inside the first split's window, and one reaching three splits
     assert bench.decode_overhead_bytes([100, 2 * 16 * 16 + 1], 32, 8, 128, 16, 16, 256) == \
         8 * (3 * 3 - 1) * 4 * rec
+
+
+def test_printed_line_stays_short():
+    """The printed line keeps the headline and every row's time, rate and traffic
+    ratio in under 9,000 characters."""
+    roof = {"bound": "hbm", "achieved": 4692.56, "peak": 8000.0, "unit": "GB/s", "frac": 0.5866,
+            "traffic": 369825607, "kernel": "sweep_ctx65536_Kauto", "algorithmic_bytes": 335125380,
+            "traffic_ratio": 1.104, "traffic_source": "profiles/pmc_summary.json"}
+    cpu = {"value": 667375.147, "unit": "tokens/s", "cores": 16, "kind": "port", "us_per_call": 1.5,
+           "sample": "x" * 120, "single_thread": {"value": 55149.7044, "unit": "tokens/s",
+                                                  "us_per_call": 18567.6, "sample": "x" * 40},
+           "affinity_cores": 16, "os_cpu_count": 16, "cpu_model": "AMD EPYC"}
+    row = {"workload": "x" * 100, "us": 1234.567, "steps": 512, "warmup": 64,
+           "spread_us": {"min_us": 1.0, "median_us": 2.0, "p99_us": 3.0, "samples": 16,
+                         "launches_per_sample": 32},
+           "tokens_per_s": 277012792.6, "GBps": 1437.14, "pct_hbm_peak": 17.96,
+           "algorithmic_bytes": 335948932, "overhead_bytes": 5744640, "poll_timeouts": 0,
+           "roofline": roof, "cpu_baseline": cpu}
+    sweep = dict({k: v for k, v in row.items() if k not in ("workload", "cpu_baseline")}, ctx=65536,
+                 splits=32, auto=False)
+    head = {"metric": "m" * 80, "value": 552.7, "roofline": roof, "cpu_baseline": cpu,
+            "config": {"workload": "x" * 200}, "decode_us": {"cold": 8.09}, "poll_timeouts": 0}
+    result = dict(head, split_sweep={"workload": "x" * 90, "rows": [sweep] * 24},
+                  **{f"row{i}": row for i in range(9)})
+    got = bench.line(result)
+    assert {k: got[k] for k in head} == head
+    assert got["row0"]["us"] == row["us"] and got["row0"]["traffic_ratio"] == 1.104
+    assert got["row0"]["cpu"] == [667375.147, "tokens/s", 16, 55149.7044]
+    assert got["split_sweep"]["rows"][0]["GBps"] == 1437.14
+    assert len(json.dumps(got)) < 9000
+    assert bench.line(dict(result, row0=dict(row, poll_timeouts=3)))["row0"]["poll_timeouts"] == 3
