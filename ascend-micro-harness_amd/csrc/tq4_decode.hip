@@ -1687,7 +1687,11 @@ hipError_t launch_fused_t(hipStream_t stream, const DecodeParams& p, size_t lds)
     // 9.1 (15.0 / 11.6), d = 128 14.8 / 11.2 (17.2 / 14.8), d = 256 27.7 / 18.9
     // (27.2 / 25.9); G = 8, d = 256 18.7 / 15.3, but 18.8 / 19.1 at K = 4, d =
     // 128 10.1 / 9.7 and 9.7 / 10.0 at K = 8, d = 64 8.5 / 8.5; G = 4 and below
-    // loses or gains nothing. The test hooks are the fused wait's.
+    // loses or gains nothing. Next to the line (2 sequences x 2 kv heads, K = 2 /
+    // 16): G = 9, d = 64 9.6 -> 8.4 / 10.6 -> 9.2, d = 128 10.5 -> 9.6 / 12.2 ->
+    // 10.4, d = 256 15.2 -> 13.4 / 20.0 -> 15.1; G = 5 at d = 256 13.0 -> 12.7 /
+    // 16.1 -> 14.4, at d = 128 9.1 -> 8.9 / 10.1 -> 9.9. The test hooks are the
+    // fused wait's.
     const bool hooks = p.withhold || p.poll_limit != kPollLimit;
     const bool wide = p.G > 8 || (D == 256 && p.G > 4 && p.K >= 8);
     if (p.K > 1 && wide && !hooks) {

@@ -113,10 +113,11 @@ __device__ __forceinline__ uint32_t level_of(float z, const LevelBin* lut)
 // 16 lanes: the two rows share the index arithmetic, the slot, the signs and
 // the scale's square root and division. Bound by the vector ALU: the codec's
 // arithmetic is about 240 instructions a row against 330 bytes of traffic at
-// d = 128. 4096 BF16 tokens x 8 heads of 128: 11.7 us with one row a lane and
-// bins of |z| (17 instructions a level), 9.1 with two rows and signed bins
-// (6 and an LDS read), 8.4 with the shared scale and a multiplier for item / H;
-// 16384 tokens 32 -> 21.5 us (3.9 TB/s).
+// d = 128. 4096 BF16 tokens x 8 heads of 128, launches in a row from a graph:
+// 11.4 us with one row a lane and bins of |z| (17 instructions a level), 9.1 with
+// two rows and signed bins (6 and an LDS read), 8.2 with the shared scale and a
+// multiplier for item / H; 1024 tokens 5.2 -> 4.4, 16384 35.8 -> 23.5 us (3.6
+// TB/s). (Eager calls over fewer buffers, 4096 tokens: 10.4 -> 7.7.)
 template <int D, int IN_BF16>
 __global__ __launch_bounds__(kRmsThreads) void rms_writer(
     const uint16_t* __restrict__ key, const uint16_t* __restrict__ value,

@@ -1,13 +1,14 @@
 // tq4_writer.hip -- reshape_and_cache for the TQ4 cache on gfx950.
 //
-// Two kernels:
-//   strip_writer     aligned 16-token strips (the reference's A8/BF16 prefill
-//                    writers, turboquant_reshape_and_cache_{a8,bf16}.cpp)
-//   scatter_writer   arbitrary slots per (request, kv_head) item, nibble-exact
-//                    read-modify-write of the value strip
-//                    (turboquant_reshape_scatter_aiv.cpp:598-731)
+// Three kernels:
+//   strip_writer          aligned 16-token strips (the reference's A8/BF16 prefill
+//                         writers, turboquant_reshape_and_cache_{a8,bf16}.cpp)
+//   scatter_writer        requests of several tokens at arbitrary slots, in chunks
+//                         of 16 tokens, nibble-exact merges into the value strips
+//                         (turboquant_reshape_scatter_aiv.cpp:598-731)
+//   scatter_token_writer  the same, one token to a request
 //
-// Work decomposition (MI355X): one 256-lane workgroup owns one strip of one
+// Work decomposition of the strip writer (MI355X): one 256-lane workgroup owns one strip of one
 // head, both planes: two panels of 16 rows x d channels, one row of each per
 // 16-lane group (two independent row jobs per lane). A row lives on 16
 // lanes with CPL = d/16 consecutive channels per lane, so the 16-point
